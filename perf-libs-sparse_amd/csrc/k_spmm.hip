@@ -4,12 +4,9 @@
 // (spmm_rowwise_csr_blocked_m_kernel, src/compressed_sparse_rows.cpp:1699-1745,
 // and the C zeroing of src/matmul.cpp:596-605): beta == 0 never reads C.
 //
-// Row-major path: a group of G lanes owns one row of C, each lane CPL of its
-// columns (k = 8: 8 x 1, so a wave covers 8 rows; k = 32: 16 x 2; k = 128:
-// 16 x 8).  For each non-zero a_p of the row the group reads the k-element row
-// B(col_p, :) as one contiguous access and accumulates alpha*a_p*B in
-// registers; C is written once.  Strided (column-major / transposed) operands
-// use the generic kernel, one thread per output element.
+// Row-major B and C: k_spmm_lds where a block of rows shares its B rows, else
+// k_spmm_gather.  Strided (column-major / transposed) operands use the generic
+// kernel, one thread per output element.
 #include <algorithm>
 #include <type_traits>
 
@@ -18,158 +15,117 @@
 
 namespace plk {
 
-template <int G, int CPL, class V, class X, bool BETA>
-__global__ __launch_bounds__(kBlock) void k_spmm_rm(
-    int32_t m, int32_t k, const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
-    const V *__restrict__ val, const X *__restrict__ B, int64_t ldb, X *__restrict__ Cm,
-    int64_t ldc, acc_t<X> alpha, acc_t<X> beta) {
-  using A = acc_t<X>;
-  const int64_t t = int64_t(xcd_swizzle(blockIdx.x, gridDim.x)) * kBlock + threadIdx.x;
-  int64_t row = t / G;
-  if (G == 64) row = __builtin_amdgcn_readfirstlane(int32_t(row));  // wave-uniform
-  const int lane = threadIdx.x & (G - 1);
-  if (row >= m) return;
-  A acc[CPL];
-#pragma unroll
-  for (int q = 0; q < CPL; ++q) acc[q] = 0;
-  const int32_t p1 = rp[row + 1];
-  // U non-zeros per step: their column/value loads issue together, then the
-  // U rows of B, so a row does not wait for one B row at a time (the last
-  // step clamps to the row's last non-zero and masks the repeats).
-  constexpr int U = CPL >= 4 ? 4 : 8;
-  for (int32_t p = rp[row]; p < p1; p += U) {
-    int32_t cc[U];
-    A a[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int32_t pp = min(p + u, p1 - 1);
-      cc[u] = ldi(ci, pp);
-      a[u] = alpha * A(ldv(val, pp));
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const X *b = B + int64_t(cc[u]) * ldb;
-      const bool ok = p + u < p1;
-#pragma unroll
-      for (int q = 0; q < CPL; ++q) {
-        const int c = lane + q * G;
-        if (c < k) {
-          const A v = a[u] * A(b[c]);
-          acc[q] += ok ? v : A(0);
-        }
-      }
-    }
-  }
-  X *crow = Cm + row * ldc;
-#pragma unroll
-  for (int q = 0; q < CPL; ++q) {
-    const int c = lane + q * G;
-    if (c < k) {
-      A r = acc[q];
-      if (BETA) r += beta * A(crow[c]);
-      crow[c] = X(r);
-    }
-  }
-}
+// Rows whose B rows are not shared within a block (scattered columns), and
+// k < 8: C rows accumulated straight from the gathered B rows.  A window of
+// G * VW columns is read by G lanes, VW adjacent columns each: 16 bytes where
+// k allows, with element alignment only, so odd k and ld take the same path
+// (the lane that would run past column k starts at k - VW and stores only its
+// own columns).  S lane groups share a row, each taking every S-th pair of
+// non-zeros, and fold with xor shuffles.  S * kGatherPairs pairs cover a row
+// of the mean length in one step (quarter or double S measured 1.2-1.9x slower
+// at k <= 16 on the 27-point stencil).  A row of more than pls::kSpmmLongRow
+// non-zeros has a workgroup of its own, the first nlong of the grid, so the
+// longest rows start first.  Bound: latency of row pointer -> entries -> B rows
+// for short products, the MALL rate of the gathered B rows for large ones
+// (power-law 262,144 rows, FP32 k = 64: 1.35 GB of B rows in 0.22 ms, 6.0
+// TB/s).  One lane group per row with 4 non-zeros in flight and scalar B loads
+// took 1.19 ms there (the longest row, ~1,100 non-zeros, outlasted the rest),
+// and row blocks staged in LDS (k <= 16) 0.36 ms against 0.067 at k = 8.
+template <int G> constexpr int kGatherPairs = G <= 2 ? 2 : 4;
 
-// Row-block variant (k < 8, or k <= 16 when the operand has no column-compressed
-// blocks): one workgroup per row block of the
-// CSR plan's nnz-balanced block table (at most kSpmmStage non-zeros and
-// kSpmmRows rows, a longer row alone in its block).  The block's column
-// indices, alpha-scaled values and row offsets are staged into LDS with
-// coalesced loads first, so the per-row loop of each lane group only waits for
-// the B rows it gathers (U rows in flight per lane), never for the matrix
-// stream.  Blocks too long to stage read the matrix from HBM directly.
-constexpr int kSpmmStage = 2048;  // = the CSR plan's row-block non-zeros (kAdaNnz)
-constexpr int kSpmmRows = 1024;   // = the CSR plan's row-block rows
-
-template <int G, int CPL, class V, class X, bool BETA>
-__global__ __launch_bounds__(kBlock) void k_spmm_blk(
-    const int32_t *__restrict__ blocks, int32_t k, const int32_t *__restrict__ rp,
+template <int G, int VW, class V, class X, bool BETA>
+__global__ __launch_bounds__(kBlock) void k_spmm_gather(
+    int32_t row0, int32_t m, int32_t k, int32_t win0, int32_t S, int32_t nlong,
+    const int32_t *__restrict__ longrow, const int32_t *__restrict__ rp,
     const int32_t *__restrict__ ci, const V *__restrict__ val, const X *__restrict__ B,
     int64_t ldb, X *__restrict__ Cm, int64_t ldc, acc_t<X> alpha, acc_t<X> beta) {
   using A = acc_t<X>;
-  __shared__ int32_t s_ci[kSpmmStage];
-  __shared__ A s_a[kSpmmStage];
-  __shared__ int32_t s_rp[kSpmmRows + 1];
-  const uint32_t blk = xcd_swizzle(blockIdx.x, gridDim.x);
-  const int tid = threadIdx.x;
-  const int32_t r0 = blocks[blk], r1 = blocks[blk + 1];
-  const int32_t e0 = rp[r0], e1 = rp[r1];
-  const int32_t nnz = e1 - e0, nrows = r1 - r0;
-  const bool staged = nnz <= kSpmmStage && nrows <= kSpmmRows;
-  if (staged) {
-    constexpr int PER = kSpmmStage / kBlock;
-    int32_t c[PER];
-    A a[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int32_t q = min(tid + u * kBlock, max(nnz - 1, 0));
-      c[u] = nnz > 0 ? ldi(ci, e0 + q) : 0;
-      a[u] = nnz > 0 ? alpha * A(ldv(val, e0 + q)) : A(0);
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int32_t q = tid + u * kBlock;
-      if (q < nnz) {
-        s_ci[q] = c[u];
-        s_a[q] = a[u];
-      }
-    }
-    for (int32_t q = tid; q <= nrows; q += kBlock) s_rp[q] = rp[r0 + q] - e0;
+  typedef X XV __attribute__((ext_vector_type(VW), aligned(sizeof(X))));
+  constexpr int U = kGatherPairs<G>;  // entry pairs in flight per lane
+  __shared__ A red[kBlock / 64][G * VW];
+  const bool whole = int32_t(blockIdx.x) < nlong;  // the workgroup shares one long row
+  const int tid = threadIdx.x, lane = tid & (G - 1);
+  if (whole) S = 64 / G;
+  const int sub = (tid & (G * S - 1)) / G;
+  int64_t row;
+  if (whole) row = longrow[blockIdx.x];
+  else row = row0 + (int64_t(xcd_swizzle(blockIdx.x - nlong, gridDim.x - nlong)) * kBlock + tid) / (G * S);
+  // the lane's first column, and where its vector starts
+  const int64_t own = int64_t(win0 + int32_t(blockIdx.y)) * (G * VW) + lane * VW;
+  const int64_t c0 = min(own, int64_t(k - VW));
+  bool live = whole || row < m;
+  uint32_t p0 = 0, p1 = 0;
+  if (live) {
+    p0 = uint32_t(rp[row]);
+    p1 = uint32_t(rp[row + 1]);
+    live = whole || p1 - p0 <= uint32_t(pls::kSpmmLongRow);  // else another workgroup's
   }
-  __syncthreads();
-  // S lane groups share a row when the block has few (long) rows, so every
-  // group has work: S = the largest power of two with nrows * S groups fitting
-  // the workgroup and G * S lanes fitting a wave; the S partial sums of a row
-  // are folded with xor shuffles inside its W = G * S lanes.
-  int S = 1;
-  while (S * 2 * G <= 64 && nrows * S * 2 <= kBlock / G) S *= 2;
-  const int W = G * S;
-  const int lane = tid & (G - 1), sub = (tid & (W - 1)) / G;
-  constexpr int U = CPL >= 4 ? 8 : 16;  // B rows in flight per lane
-  for (int32_t rr = tid / W; rr < nrows; rr += kBlock / W) {
-    const int32_t p0 = staged ? s_rp[rr] : rp[r0 + rr] - e0;
-    const int32_t p1 = staged ? s_rp[rr + 1] : rp[r0 + rr + 1] - e0;
-    A acc[CPL];
+  A acc[VW];
 #pragma unroll
-    for (int q = 0; q < CPL; ++q) acc[q] = 0;
-    for (int32_t p = p0 + sub; p < p1; p += U * S) {
-      int32_t cc[U];
-      A a[U];
+  for (int t = 0; t < VW; ++t) acc[t] = A(0);
+  if (live && p0 < p1) {
+    // entries in aligned pairs (one 8-byte index load, one 2-value load; the
+    // plan's arrays end with one padding entry), those outside the row masked
+    const uint32_t step = 2 * (whole ? S * (kBlock / 64) : S), last = (p1 - 1) & ~1u;
+    const X *Bc = B + c0;
+    for (uint32_t p = (p0 & ~1u) + 2 * (sub + (whole ? (tid >> 6) * S : 0)); p < p1;
+         p += U * step) {
+      int32_t c[U][2];
+      A a[U][2];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int32_t pp = min(p + u * S, p1 - 1);
-        cc[u] = staged ? s_ci[pp] : ldi(ci, e0 + pp);
-        a[u] = staged ? s_a[pp] : alpha * A(ldv(val, e0 + pp));
-      }
+      for (int u = 0; u < U; ++u) ld_pair(ci, val, int32_t(min(p + u * step, last)), c[u], a[u]);
+      XV b[U][2];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const X *b = B + int64_t(cc[u]) * ldb;
-        const bool ok = p + u * S < p1;
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int q = 0; q < CPL; ++q) {
-          const int col = lane + q * G;
-          if (col < k) {
-            const A v = a[u] * A(b[col]);
-            acc[q] += ok ? v : A(0);
-          }
+        for (int h = 0; h < 2; ++h)
+          b[u][h] = *reinterpret_cast<const XV *>(Bc + int64_t(c[u][h]) * ldb);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t q = p + u * step + h;
+          const bool ok = q >= p0 && q < p1;
+          const A w = alpha * a[u][h];
+#pragma unroll
+          for (int t = 0; t < VW; ++t) acc[t] = ok ? acc[t] + w * A(b[u][h][t]) : acc[t];
         }
-      }
     }
-    for (int o = G; o < W; o <<= 1)  // all W lanes of the row take this path together
+  }
+  for (int o = G; o < G * S; o <<= 1)
 #pragma unroll
-      for (int q = 0; q < CPL; ++q) acc[q] += __shfl_xor(acc[q], o);
-    X *crow = Cm + int64_t(r0 + rr) * ldc;
+    for (int t = 0; t < VW; ++t) acc[t] += __shfl_xor(acc[t], o);
+  if (whole) {
+    if (sub == 0)
 #pragma unroll
-    for (int q = 0; q < CPL; ++q) {
-      const int col = lane + q * G;
-      if (sub == 0 && col < k) {
-        A r = acc[q];
-        if (BETA) r += beta * A(crow[col]);
-        crow[col] = X(r);
-      }
+      for (int t = 0; t < VW; ++t) red[tid >> 6][lane * VW + t] = acc[t];
+    __syncthreads();
+    if (tid >= G) return;
+#pragma unroll
+    for (int t = 0; t < VW; ++t)
+      acc[t] = (red[0][lane * VW + t] + red[1][lane * VW + t]) +
+               (red[2][lane * VW + t] + red[3][lane * VW + t]);
+  }
+  if (!live || sub != 0 || own >= k) return;
+  X *c = Cm + row * ldc + c0;
+  if (c0 == own) {
+    XV o;
+    if (BETA) o = *reinterpret_cast<const XV *>(c);
+#pragma unroll
+    for (int t = 0; t < VW; ++t) {
+      A r = acc[t];
+      if (BETA) r += beta * A(o[t]);
+      o[t] = X(r);
     }
+    *reinterpret_cast<XV *>(c) = o;
+  } else {
+#pragma unroll
+    for (int t = 0; t < VW; ++t)
+      if (c0 + t >= own) {
+        A r = acc[t];
+        if (BETA) r += beta * A(c[t]);
+        c[t] = X(r);
+      }
   }
 }
 
@@ -640,34 +596,51 @@ __global__ __launch_bounds__(kBlock) void k_strided_copy(int64_t n, const X *src
 }
 
 namespace {
-template <int G, int CPL, class V, class X>
-void launch_rm(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
-               double beta, void *C, int64_t ldc, hipStream_t s) {
-  // Narrow B (k <= 16; k >= 8 only without column-compressed blocks): the
-  // row-block kernel over the plan's block table.
-  // Wider B rows keep one row per lane group and far more rows in flight
-  // (measured faster for k = 32 and 128 on the 27-point stencil).
-  if (A.nblocks > 0 && G * CPL <= 16) {
-    if (beta != 0.0)
-      k_spmm_blk<G, CPL, V, X, true><<<A.nblocks, kBlock, 0, s>>>(
-          A.blocks.as<int32_t>(), k, A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(),
-          (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(beta));
-    else
-      k_spmm_blk<G, CPL, V, X, false><<<A.nblocks, kBlock, 0, s>>>(
-          A.blocks.as<int32_t>(), k, A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(),
-          (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(0));
-    return;
-  }
-  const unsigned grid = grid_for(int64_t(A.m) * G);
-  if (grid == 0) return;
-  if (beta != 0.0)
-    k_spmm_rm<G, CPL, V, X, true><<<grid, kBlock, 0, s>>>(
-        A.m, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, ldb,
-        (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(beta));
-  else
-    k_spmm_rm<G, CPL, V, X, false><<<grid, kBlock, 0, s>>>(
-        A.m, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, ldb,
-        (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(0));
+template <int G, int VW, class V, class X>
+void launch_gather(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
+                   double beta, void *C, int64_t ldc, hipStream_t s) {
+  const double mean = double(A.nnz) / A.m;
+  int32_t S = 1;  // lane groups per row
+  while (2 * S * G <= 64 && 2 * kGatherPairs<G> * S <= mean) S *= 2;
+  const int64_t windows = (int64_t(k) + G * VW - 1) / (G * VW);
+  const int32_t slice = (1 << 30) / (G * S);  // rows per launch: fewer than 2^32 threads
+  auto go = [&](auto kern) {
+    for (int64_t w = 0; w < windows; w += 65535)
+      for (int64_t r = 0; r < A.m; r += slice) {
+        const int32_t rows = int32_t(std::min<int64_t>(slice, A.m - r)), nl = r == 0 ? A.nlong : 0;
+        const dim3 grid(unsigned(nl) + grid_for(int64_t(rows) * (G * S)),
+                        unsigned(std::min<int64_t>(65535, windows - w)));
+        kern<<<grid, kBlock, 0, s>>>(int32_t(r), int32_t(r) + rows, k, int32_t(w), S, nl,
+                                     A.longrow.as<int32_t>(), A.rp.as<int32_t>(),
+                                     A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, ldb, (X *)C,
+                                     ldc, acc_t<X>(alpha), acc_t<X>(beta));
+      }
+  };
+  if (beta != 0.0) go(k_spmm_gather<G, VW, V, X, true>);
+  else go(k_spmm_gather<G, VW, V, X, false>);
+}
+
+template <int VW, class V, class X>
+void gather_lanes(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
+                  double beta, void *C, int64_t ldc, hipStream_t s) {
+  const int32_t lanes = (k + VW - 1) / VW;
+  if (lanes <= 1) launch_gather<1, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else if (lanes <= 2) launch_gather<2, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else if (lanes <= 4) launch_gather<4, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else if (lanes <= 8) launch_gather<8, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else if (lanes <= 16) launch_gather<16, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else if (lanes <= 32) launch_gather<32, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else launch_gather<64, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+}
+
+// VW: 16 bytes of columns per lane, fewer when B has fewer columns.
+template <class V, class X>
+void dispatch_gather(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
+                     double beta, void *C, int64_t ldc, hipStream_t s) {
+  if (sizeof(X) == 4 && k >= 4)
+    gather_lanes<(sizeof(X) == 4 ? 4 : 2), V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else if (k >= 2) gather_lanes<2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  else launch_gather<1, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
 }
 
 template <class V, class X>
@@ -721,23 +694,6 @@ void launch_lds(const pls::DevCsr &A, int32_t k, double alpha, const void *B, in
   }
 }
 
-template <class V, class X>
-void dispatch_rm(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
-                 double beta, void *C, int64_t ldc, hipStream_t s) {
-  if (k <= 1) launch_rm<1, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 2) launch_rm<2, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 4) launch_rm<4, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 8) launch_rm<8, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 16) launch_rm<16, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  // wide B: several columns per lane keep more rows in flight per wave
-  // (measured on the 27-point stencil: k = 32 as 16 x 2 and k = 128 as 16 x 8
-  // beat one or two columns per lane by 1.2x and 1.1-1.25x)
-  else if (k <= 32) launch_rm<16, 2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 64) launch_rm<16, 4, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 128) launch_rm<16, 8, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k <= 256) launch_rm<32, 8, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else launch_rm<64, 8, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-}
 }  // namespace
 
 hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, const void *B,
@@ -750,10 +706,7 @@ hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, con
     if (b_sc == 1 && c_sc == 1 && k >= 8 && A.lb_state == 1 && A.lb_nblocks > 0) {
       launch_lds<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
     } else if (b_sc == 1 && c_sc == 1) {
-      // row-major: column slices of at most 512 (the widest lane-group shape)
-      for (int32_t c0 = 0; c0 < k; c0 += 512)
-        dispatch_rm<V, X>(A, std::min<int32_t>(512, k - c0), alpha, static_cast<const X *>(B) + c0,
-                          b_sr, beta, static_cast<X *>(C) + c0, c_sr, s);
+      dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
     } else {
       const unsigned grid = grid_for(int64_t(A.m) * k);
       if (beta != 0.0)

@@ -204,6 +204,12 @@ static perflibs_status_t build_csr_plan(perflibs_spmat_top_t *A, const Operand &
     }
     d->nblocks = int32_t(blocks.size() - 1);
     e = d->blocks.upload(blocks.data(), sizeof(int32_t) * blocks.size());
+    std::vector<int32_t> longrow;
+    for (int32_t i = 0; i < o.m; ++i)
+      if (o.prp[i + 1] - o.prp[i] > kSpmmLongRow) longrow.push_back(i);
+    d->nlong = int32_t(longrow.size());
+    if (e == hipSuccess && d->nlong > 0)
+      e = d->longrow.upload(longrow.data(), sizeof(int32_t) * longrow.size());
   }
   if (e != hipSuccess) return hip_fail(A, e, "CSR plan upload");
   A->plan.clear();

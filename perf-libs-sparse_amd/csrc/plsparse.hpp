@@ -99,6 +99,10 @@ struct Dense {
 };
 
 // Device CSR (0-based) with the row-block table of the adaptive kernel.
+// Non-zeros of a row above which k_spmm_gather gives it a workgroup of its own
+// (power-law 1M rows, FP64 k = 8 / 64: 411 / 1702 us with 128, 387 / 1608 with
+// 256, 380 / 1577 with 512).
+constexpr int32_t kSpmmLongRow = 512;
 struct DevCsr {
   int32_t m = 0, n = 0;
   int64_t nnz = 0;
@@ -107,6 +111,8 @@ struct DevCsr {
   DevBuf blocks;  // int32 row starts of nnz-balanced row blocks (+ final m)
   int32_t nblocks = 0;
   int32_t vec_lanes = 8;  // lanes per row of the CSR-vector kernel
+  DevBuf longrow;         // int32 [nlong] rows of more than kSpmmLongRow non-zeros
+  int32_t nlong = 0;
   // Column-compressed row blocks of the wide-B SpMM kernel (built on the first
   // SpMM with k >= 8, spmm_blocks.cpp): each block of rows lists its distinct
   // columns once (ucol), and each non-zero stores its column's position in
