@@ -148,7 +148,8 @@ perflibs_status_t to_csr_keeping_blocks(perflibs_spmat_top_t *A, bool keep) {
 }
 
 // CSR plan of op(A) for SpMM with k columns of B; for k >= 8 also the
-// column-compressed row blocks of the wide-B kernel (built once per plan).
+// column-compressed row blocks (cut once per plan) in the form that product
+// runs on.
 perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k) {
   pls::Operand o;
   if (!(A->plan.csr && A->plan.op == op)) {
@@ -156,10 +157,14 @@ perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k) {
     const perflibs_status_t st = pls::build_plan(A, o, op, PERFLIBS_AMD_CSR_VECTOR);
     if (st != PERFLIBS_STATUS_SUCCESS) return st;
   }
-  if (k >= 8 && A->plan.csr->lb_state == 0) {
+  pls::DevCsr &d = *A->plan.csr;
+  if (k < 8 || d.lb_state < 0) return PERFLIBS_STATUS_SUCCESS;
+  auto tiles = [&] { return pls::spmm_on_tiles(d, A->dt == DType::F64, k); };
+  if (d.lb_state == 0 || (tiles() ? d.ntiles < 0 : !d.lb_lds)) {
     if (!o.prp && !pls::make_operand(A, op, o))
       return pls::exec_fail(A, "matrix format has no GPU SpMM path");
-    const hipError_t e = pls::build_spmm_blocks(o, *A->plan.csr, A->spmm_rows);
+    if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);
+    const hipError_t e = pls::upload_spmm_form(o, d, tiles());
     if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM block upload");
   }
   return PERFLIBS_STATUS_SUCCESS;

@@ -4,8 +4,8 @@
 // (spmm_rowwise_csr_blocked_m_kernel, src/compressed_sparse_rows.cpp:1699-1745,
 // and the C zeroing of src/matmul.cpp:596-605): beta == 0 never reads C.
 //
-// Row-major B and C: k_spmm_lds where a block of rows shares its B rows, else
-// k_spmm_gather.  Strided (column-major / transposed) operands use the generic
+// Row-major B and C: k_spmm_tile or k_spmm_lds where a block of rows shares its
+// B rows, else k_spmm_gather.  Strided (column-major / transposed) operands use the generic
 // kernel, one thread per output element.
 #include <algorithm>
 #include <type_traits>
@@ -129,16 +129,214 @@ __global__ __launch_bounds__(kBlock) void k_spmm_gather(
   }
 }
 
-// Column-compressed row blocks (dispatched for k >= 8 when the plan's block
-// lists are short enough, see build_spmm_blocks): one workgroup per block of
+// VW columns of one C row from column c0 on; the lane owns those from `own` on.
+template <int VW, class X, bool BETA>
+__device__ __forceinline__ void store_cols(X *crow, int64_t c0, int64_t own, int32_t k,
+                                           const acc_t<X> (&v)[VW], acc_t<X> alpha,
+                                           acc_t<X> beta) {
+  using A = acc_t<X>;
+  typedef X XV __attribute__((ext_vector_type(VW), aligned(sizeof(X))));
+  if (own >= k) return;
+  X *c = crow + c0;
+  if (c0 == own) {
+    XV o;
+    if (BETA) o = *reinterpret_cast<const XV *>(c);
+#pragma unroll
+    for (int t = 0; t < VW; ++t) {
+      A r = alpha * v[t];
+      if (BETA) r += beta * A(o[t]);
+      o[t] = X(r);
+    }
+    *reinterpret_cast<XV *>(c) = o;
+  } else {
+#pragma unroll
+    for (int t = 0; t < VW; ++t)
+      if (c0 + t >= own) {
+        A r = alpha * v[t];
+        if (BETA) r += beta * A(c[t]);
+        c[t] = X(r);
+      }
+  }
+}
+
+// Row tiles (pls::spmm_on_tiles: operands whose rows share columns, k > 16): one
+// wave multiplies a tile of up to 32 rows, two halves of 16, by a window of NW *
+// 16 * VW columns of B on the matrix cores.  The tile's distinct columns are
+// listed four to a step; a step's B rows are read once, VW adjacent columns per
+// lane (the columns of a window are permuted), and serve both halves through
+// v_mfma_f64_16x16x4 / v_mfma_f32_16x16x4.  The values stay compressed: per step
+// and half the non-zero ones in lane order behind a 64-bit mask of the lanes
+// that have one.  They are copied to the wave's LDS slice with full-width loads
+// one group of G steps ahead, and each lane picks its own by counting mask bits
+// (picked straight from global memory, and with 16 rows per tile, the texture
+// path was busy 74% of the kernel and FP64 k = 32 took 129 us below).  Columns
+// of one half alone come first and last, so those steps skip the other half.
+// Windows are the slow grid index and the grid a multiple of 8, so an XCD sweeps
+// its own tiles one window at a time and the B rows of a sweep stay in its L2
+// (two windows at k = 128 side by side: 446 us against 421).
+// Bound: 27-point stencil 96^3, FP64 k = 32, 203 us (floor 156 at the copy rate,
+// matrix cores 106), k = 128 on 80^3 408 us (floor 257): matrix cores about half
+// busy and 2.5 GB moved for 1.2 GB, B rows fetched again across grid planes.
+// k_spmm_lds takes 275 and 553 us there.
+// A wave whose results hold a NaN computes them again entry by entry: a column
+// some row of the tile does not have is multiplied by zero for that row, which
+// changes nothing unless the B value is infinite or NaN.
+template <class X> struct TileAcc;
+template <> struct TileAcc<double> {
+  typedef double T __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ T mma(double a, double b, T c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int kk, int r) { return 4 * r + kk; }
+};
+template <> struct TileAcc<float> {
+  typedef float T __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ T mma(float a, float b, T c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int kk, int r) { return 4 * kk + r; }
+};
+
+template <class V, class X>
+__device__ __noinline__ acc_t<X> csr_dot(int32_t p0, int32_t p1, int64_t c, const int32_t *ci,
+                                         const V *val, const X *Bm, int64_t ldb) {
+  acc_t<X> s = 0;
+  for (int32_t p = p0; p < p1; ++p)
+    s += acc_t<X>(ldv(val, p)) * acc_t<X>(Bm[int64_t(ci[p]) * ldb + c]);
+  return s;
+}
+
+template <int NW, int VW, class V, class X, bool BETA>
+__global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
+    int32_t tile0, int32_t ntiles, int32_t win0, int32_t k, const pls::SpmmTile *__restrict__ tiles,
+    const int32_t *__restrict__ trow, const uint64_t *__restrict__ mask,
+    const int32_t *__restrict__ tcol, const V *__restrict__ tval, const int32_t *__restrict__ rp,
+    const int32_t *__restrict__ ci, const V *__restrict__ val, const X *__restrict__ Bm,
+    int64_t ldb, X *__restrict__ Cm, int64_t ldc, acc_t<X> alpha, acc_t<X> beta) {
+  using A = acc_t<X>;
+  using M = TileAcc<X>;
+  typedef X XV __attribute__((ext_vector_type(VW), aligned(sizeof(X))));
+  constexpr int G = 4;       // steps in flight
+  constexpr int PF = G / 2;  // prefetched value registers: 64 values each
+  __shared__ A lds[kBlock / 64][G * 128];  // the values of G steps
+  const int lane = threadIdx.x & 63, n = lane & 15, kk = lane >> 4;
+  A *av = lds[threadIdx.x >> 6];
+  const int32_t tile = tile0 + int32_t(xcd_swizzle(blockIdx.x, gridDim.x)) * (kBlock / 64) +
+                       __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (tile >= ntiles) return;
+  const int32_t pass = win0 + int32_t(blockIdx.y);
+  const pls::SpmmTile t0 = tiles[tile], t1 = tiles[tile + 1];
+  int64_t own[NW], c0[NW];
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    own[w] = (int64_t(pass) * NW + w) * (16 * VW) + n * VW;
+    c0[w] = min(own[w], int64_t(k - VW));
+  }
+  typename M::T acc[2][NW][VW];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+      for (int e = 0; e < VW; ++e) acc[h][w][e] = typename M::T{0, 0, 0, 0};
+  const V *tv = tval + t0.val0;
+  const uint32_t ld = uint32_t(ldb);
+  A pf[PF];
+#pragma unroll
+  for (int i = 0; i < PF; ++i) pf[i] = A(ldv(tv, lane + 64 * i));
+  for (int32_t q0 = t0.step0; q0 < t1.step0; q0 += 16) {
+    // columns of the next 16 steps, one per lane (past the last: the last
+    // one), and their masks, two per step (past the last: 0)
+    const int32_t ns = min(t1.step0 - q0, 16);
+    const int32_t cv = ldi(tcol, 4 * int64_t(q0) + min(lane, 4 * ns - 1));
+    const uint64_t mv = lane < 2 * ns ? mask[2 * int64_t(q0) + lane] : 0;
+    for (int32_t s = 0; s < ns; s += G) {
+      XV b[G][NW];
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        const uint32_t col = __builtin_amdgcn_ds_bpermute(kk * 4 + s * 16 + u * 16, cv);
+        const X *bp = Bm + uint64_t(col) * ld;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) b[u][w] = *reinterpret_cast<const XV *>(bp + c0[w]);
+      }
+      uint64_t m[G][2];
+      int32_t nv = 0;
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(mv >> 32), 2 * (s + u) + h),
+                         lo = __builtin_amdgcn_readlane(uint32_t(mv), 2 * (s + u) + h);
+          m[u][h] = uint64_t(hi) << 32 | lo;
+          nv += __builtin_popcountll(m[u][h]);
+        }
+#pragma unroll
+      for (int i = 0; i < PF; ++i) av[lane + 64 * i] = pf[i];
+      for (int32_t i = 64 * PF; i < nv; i += 64) av[lane + i] = A(ldv(tv, lane + i));
+      tv += nv;
+#pragma unroll
+      for (int i = 0; i < PF; ++i) pf[i] = A(ldv(tv, lane + 64 * i));
+      __builtin_amdgcn_wave_barrier();
+      const A *ap = av;
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          if (m[u][h] == 0) continue;
+          A a = ap[__builtin_amdgcn_mbcnt_hi(uint32_t(m[u][h] >> 32),
+                                             __builtin_amdgcn_mbcnt_lo(uint32_t(m[u][h]), 0))];
+          a = __builtin_amdgcn_inverse_ballot_w64(m[u][h]) ? a : A(0);
+          ap += __builtin_popcountll(m[u][h]);
+#pragma unroll
+          for (int w = 0; w < NW; ++w)
+#pragma unroll
+            for (int e = 0; e < VW; ++e) acc[h][w][e] = M::mma(a, A(b[u][w][e]), acc[h][w][e]);
+        }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  bool nan = false;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+      for (int e = 0; e < VW; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) nan = nan || acc[h][w][e][r] != acc[h][w][e][r];
+  const bool redo = __any(nan);
+  const int32_t nrows = t1.row0 - t0.row0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int32_t i = M::row(kk, r) + (h ? t0.half : 0);
+      if (i >= (h ? nrows : t0.half)) continue;
+      const int32_t row = trow[t0.row0 + i];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        A out[VW];
+#pragma unroll
+        for (int e = 0; e < VW; ++e) out[e] = acc[h][w][e][r];
+        if (redo)
+          for (int e = 0; e < VW; ++e)
+            out[e] = csr_dot<V, X>(rp[row], rp[row + 1], c0[w] + e, ci, val, Bm, ldb);
+        store_cols<VW, X, BETA>(Cm + int64_t(row) * ldc, c0[w], own[w], k, out, alpha, beta);
+      }
+    }
+}
+
+// Column-compressed row blocks (k >= 8 when the plan's block lists are short
+// enough, see build_spmm_blocks, and the product is not one for the row tiles
+// above): one workgroup per block of
 // rows, consecutive ones or (brow != nullptr) the rows brow lists for the
 // block, whose non-zeros the plan keeps in block order (prp, lval, lidx: one
 // contiguous range per block, like consecutive rows).  The block's
 // alpha-scaled values and one-byte list positions are staged in LDS once (in
 // aligned pairs); then, KC columns at a time, every B row the block needs is
 // loaded into LDS once (coalesced, KC contiguous elements per row, 16 bytes per
-// lane when VB) and each row of C is accumulated from LDS by a group of
-// KC / CPL lanes (CPL adjacent columns each, written as one vector when VB),
+// lane) and each row of C is accumulated from LDS by a group of
+// KC / CPL lanes (CPL adjacent columns each, written as one vector),
 // 8 non-zeros in flight per lane.  On the 27-point stencil a staged B row
 // feeds about 5 non-zeros of a block of clustered rows (2.6 with consecutive
 // rows), so L2 -> CU traffic for B falls by that factor against the direct
@@ -146,7 +344,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_gather(
 // with more than UMAX distinct columns or lb_nnz_per_ucol(UMAX) * UMAX
 // non-zeros) spreads its non-zeros over the workgroup's lane groups, reads B
 // directly and sums the groups through LDS.
-template <int KC, int UMAX, int CPL, class V, class X, bool BETA, bool VB>
+template <int KC, int UMAX, int CPL, class V, class X, bool BETA>
 __global__ __launch_bounds__(kBlock) void k_spmm_lds(
     const int32_t *__restrict__ row0s, const int32_t *__restrict__ uoff,
     const int32_t *__restrict__ ucol, const uint8_t *__restrict__ lidx,
@@ -156,9 +354,6 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
     int64_t ldb, X *__restrict__ Cm, int64_t ldc, acc_t<X> alpha, acc_t<X> beta) {
   using A = acc_t<X>;
   constexpr int NG = kBlock / KC;  // lane groups (rows in flight) per workgroup
-  // B rows in flight per thread while staging: up to 8, at most the list rows
-  // a thread stages
-  constexpr int NIF = UMAX / NG < 8 ? UMAX / NG : 8;
   __shared__ __align__(16) A sB[UMAX * KC];
   __shared__ A s_a[pls::lb_nnz_per_ucol(UMAX) * UMAX];
   __shared__ uint8_t s_l[pls::lb_nnz_per_ucol(UMAX) * UMAX];
@@ -233,13 +428,14 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
   while (S * 2 * G <= 64 && nrows * S * 2 <= NGC) S *= 2;
   const int lc = tid % G, sub = (tid % (G * S)) / G;
   for (int32_t c0 = 0; c0 < k; c0 += KC) {
-    if constexpr (VB) {
-      // B rows of the list, columns [c0, c0 + KC), 16 bytes per lane (B and
-      // its rows 16-byte aligned): half (FP64) or a quarter (FP32) of the
-      // load instructions of one element per lane
+    {
+      // B rows of the list, columns [c0, c0 + KC), 16 bytes per lane with
+      // element alignment only: half (FP64) or a quarter (FP32) of the load
+      // instructions of one element per lane
       constexpr int VW = 16 / sizeof(X), LR = KC / VW, NGV = kBlock / LR;
       constexpr int NIFV = UMAX / NGV < 1 ? 1 : UMAX / NGV < 8 ? UMAX / NGV : 8;
       typedef X XV __attribute__((ext_vector_type(VW)));
+      typedef X XU __attribute__((ext_vector_type(VW), aligned(sizeof(X))));
       const int lv = tid % LR;
       const int32_t cv = c0 + lv * VW;
       const bool full = cv + VW <= k;
@@ -249,7 +445,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
         for (int s = 0; s < NIFV; ++s) {
           const X *src = B + int64_t(s_uc[min(i0 + s * NGV, nu - 1)]) * ldb + cv;
           if (full) {
-            t[s] = *reinterpret_cast<const XV *>(src);
+            t[s] = *reinterpret_cast<const XU *>(src);
           } else {
 #pragma unroll
             for (int e = 0; e < VW; ++e) t[s][e] = cv + e < k ? src[e] : X(0);
@@ -258,21 +454,6 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
 #pragma unroll
         for (int s = 0; s < NIFV; ++s)
           if (i0 + s * NGV < nu) *reinterpret_cast<XV *>(&sB[(i0 + s * NGV) * KC + lv * VW]) = t[s];
-      }
-    } else {
-      const int32_t col = c0 + lane;
-      // B rows of the list, columns [c0, c0 + KC): NG rows per pass, NIF passes
-      // of loads in flight before their LDS stores
-      for (int32_t i0 = grp; i0 < nu; i0 += NIF * NG) {
-        A t[NIF];
-#pragma unroll
-        for (int s = 0; s < NIF; ++s) {
-          const int32_t i = min(i0 + s * NG, nu - 1);
-          t[s] = col < k ? A(B[int64_t(s_uc[i]) * ldb + col]) : A(0);
-        }
-#pragma unroll
-        for (int s = 0; s < NIF; ++s)
-          if (i0 + s * NG < nu) sB[(i0 + s * NG) * KC + lane] = t[s];
       }
     }
     __syncthreads();
@@ -312,8 +493,8 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
       if (sub == 0) {
         X *c = Cm + int64_t(brow ? s_row[rr] : r0 + rr) * ldc;
         const int32_t cb = c0 + lc * CPL;
-        if (VB && cb + CPL <= k) {  // the lane's CPL columns as one vector (C aligned like B)
-          typedef X XC __attribute__((ext_vector_type(CPL)));
+        if (cb + CPL <= k) {  // the lane's CPL columns as one vector
+          typedef X XC __attribute__((ext_vector_type(CPL), aligned(sizeof(X))));
           XC o;
           if (BETA) o = *reinterpret_cast<const XC *>(c + cb);
 #pragma unroll
@@ -486,36 +667,6 @@ __device__ __forceinline__ void ld_adjacent(const V *p, float (&x)[N]) {
       if constexpr (sizeof(V) == 2) x[i] = __uint_as_float(uint32_t(V(t[i])) << 16);
       else x[i] = t[i];
     }
-  }
-}
-
-// VW columns of one C row from column c0 on; the lane owns those from `own` on.
-template <int VW, class X, bool BETA>
-__device__ __forceinline__ void store_cols(X *crow, int64_t c0, int64_t own, int32_t k,
-                                           const acc_t<X> (&v)[VW], acc_t<X> alpha,
-                                           acc_t<X> beta) {
-  using A = acc_t<X>;
-  typedef X XV __attribute__((ext_vector_type(VW), aligned(sizeof(X))));
-  if (own >= k) return;
-  X *c = crow + c0;
-  if (c0 == own) {
-    XV o;
-    if (BETA) o = *reinterpret_cast<const XV *>(c);
-#pragma unroll
-    for (int t = 0; t < VW; ++t) {
-      A r = alpha * v[t];
-      if (BETA) r += beta * A(o[t]);
-      o[t] = X(r);
-    }
-    *reinterpret_cast<XV *>(c) = o;
-  } else {
-#pragma unroll
-    for (int t = 0; t < VW; ++t)
-      if (c0 + t >= own) {
-        A r = alpha * v[t];
-        if (BETA) r += beta * A(c[t]);
-        c[t] = X(r);
-      }
   }
 }
 
@@ -861,7 +1012,10 @@ __global__ __launch_bounds__(kBlock) void k_strided_copy(int64_t n, const X *src
 namespace {
 template <int G, int VW, class V, class X>
 void launch_gather(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
-                   double beta, void *C, int64_t ldc, hipStream_t s) {
+                   double beta, void *C, int64_t ldc, hipStream_t s, bool direct) {
+  // direct: only the rows that the tiles leave out, a workgroup each
+  const int32_t m = direct ? 0 : A.m, nlong = direct ? A.t_ndirect : A.nlong;
+  const int32_t *longrow = (direct ? A.t_direct : A.longrow).template as<int32_t>();
   const double mean = double(A.nnz) / A.m;
   int32_t S = 1;  // lane groups per row
   while (2 * S * G <= 64 && 2 * kGatherPairs<G> * S <= mean) S *= 2;
@@ -869,14 +1023,15 @@ void launch_gather(const pls::DevCsr &A, int32_t k, double alpha, const void *B,
   const int32_t slice = (1 << 30) / (G * S);  // rows per launch: fewer than 2^32 threads
   auto go = [&](auto kern) {
     for (int64_t w = 0; w < windows; w += 65535)
-      for (int64_t r = 0; r < A.m; r += slice) {
-        const int32_t rows = int32_t(std::min<int64_t>(slice, A.m - r)), nl = r == 0 ? A.nlong : 0;
+      for (int64_t r = 0; r < std::max(m, 1); r += slice) {
+        const int32_t rows = int32_t(std::min<int64_t>(slice, m - r)), nl = r == 0 ? nlong : 0;
         const dim3 grid(unsigned(nl) + grid_for(int64_t(rows) * (G * S)),
                         unsigned(std::min<int64_t>(65535, windows - w)));
-        kern<<<grid, kBlock, 0, s>>>(int32_t(r), int32_t(r) + rows, k, int32_t(w), S, nl,
-                                     A.longrow.as<int32_t>(), A.rp.as<int32_t>(),
-                                     A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, ldb, (X *)C,
-                                     ldc, acc_t<X>(alpha), acc_t<X>(beta));
+        if (grid.x == 0) continue;
+        kern<<<grid, kBlock, 0, s>>>(int32_t(r), int32_t(r) + rows, k, int32_t(w), S, nl, longrow,
+                                     A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(),
+                                     (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha),
+                                     acc_t<X>(beta));
       }
   };
   if (beta != 0.0) go(k_spmm_gather<G, VW, V, X, true>);
@@ -885,25 +1040,61 @@ void launch_gather(const pls::DevCsr &A, int32_t k, double alpha, const void *B,
 
 template <int VW, class V, class X>
 void gather_lanes(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
-                  double beta, void *C, int64_t ldc, hipStream_t s) {
+                  double beta, void *C, int64_t ldc, hipStream_t s, bool direct) {
   const int32_t lanes = (k + VW - 1) / VW;
-  if (lanes <= 1) launch_gather<1, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (lanes <= 2) launch_gather<2, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (lanes <= 4) launch_gather<4, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (lanes <= 8) launch_gather<8, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (lanes <= 16) launch_gather<16, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (lanes <= 32) launch_gather<32, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else launch_gather<64, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  if (lanes <= 1) launch_gather<1, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else if (lanes <= 2) launch_gather<2, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else if (lanes <= 4) launch_gather<4, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else if (lanes <= 8) launch_gather<8, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else if (lanes <= 16) launch_gather<16, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else if (lanes <= 32) launch_gather<32, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else launch_gather<64, VW, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
 }
 
 // VW: 16 bytes of columns per lane, fewer when B has fewer columns.
 template <class V, class X>
 void dispatch_gather(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
-                     double beta, void *C, int64_t ldc, hipStream_t s) {
+                     double beta, void *C, int64_t ldc, hipStream_t s, bool direct) {
   if (sizeof(X) == 4 && k >= 4)
-    gather_lanes<(sizeof(X) == 4 ? 4 : 2), V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else if (k >= 2) gather_lanes<2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
-  else launch_gather<1, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+    gather_lanes<(sizeof(X) == 4 ? 4 : 2), V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else if (k >= 2) gather_lanes<2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+  else launch_gather<1, 1, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, direct);
+}
+
+template <int NW, int VW, class V, class X>
+void launch_tile(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
+                 double beta, void *C, int64_t ldc, hipStream_t s) {
+  constexpr int WCOLS = 16 * VW * NW;  // columns of one wave
+  const int64_t windows = (int64_t(k) + WCOLS - 1) / WCOLS;
+  const int64_t slice = int64_t(1) << 25;  // tiles per launch
+  auto go = [&](auto kern) {
+    for (int64_t w = 0; w < windows; w += 65535)
+      for (int64_t t = 0; t < A.ntiles; t += slice) {
+        const int32_t n = int32_t(std::min(slice, A.ntiles - t));
+        // a multiple of 8 workgroups per window: a tile's windows run on one XCD
+        const dim3 grid((grid_for(int64_t(n) * 64) + 7) / 8 * 8,
+                        unsigned(std::min<int64_t>(65535, windows - w)));
+        kern<<<grid, kBlock, 0, s>>>(
+            int32_t(t), int32_t(t) + n, int32_t(w), k, A.t_tiles.as<pls::SpmmTile>(), A.t_row.as<int32_t>(),
+            A.t_mask.as<uint64_t>(), A.t_col.as<int32_t>(), A.t_val.as<V>(), A.rp.as<int32_t>(),
+            A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha),
+            acc_t<X>(beta));
+      }
+  };
+  if (beta != 0.0) go(k_spmm_tile<NW, VW, V, X, true>);
+  else go(k_spmm_tile<NW, VW, V, X, false>);
+}
+template <class V, class X>
+void dispatch_tile(const pls::DevCsr &A, int32_t k, double alpha, const void *B, int64_t ldb,
+                   double beta, void *C, int64_t ldc, hipStream_t s) {
+  if constexpr (sizeof(X) == 8) {
+    if (k <= 32) launch_tile<1, 2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+    else launch_tile<2, 2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  } else {
+    if (k <= 32) launch_tile<1, 2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+    else if (k <= 64) launch_tile<1, 4, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+    else launch_tile<2, 4, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+  }
 }
 
 template <class V, class X>
@@ -920,23 +1111,14 @@ void launch_lds(const pls::DevCsr &A, int32_t k, double alpha, const void *B, in
     const auto *brow = A.lb_brow.as<int32_t>();
     const auto *prp = A.lb_prp.as<int32_t>();
     const auto *lval = A.lb_val.as<V>();
-    // 16-byte B staging loads and vector C rows when B, C and their rows are
-    // 16-byte aligned
-    const bool vb = (reinterpret_cast<uintptr_t>(B) & 15) == 0 && (ldb * int64_t(sizeof(X))) % 16 == 0 &&
-                    (reinterpret_cast<uintptr_t>(C) & 15) == 0 && (ldc * int64_t(sizeof(X))) % 16 == 0;
-    auto launch = [&](auto vtag) {
-      constexpr bool VB = decltype(vtag)::value;
-      if (beta != 0.0)
-        k_spmm_lds<KC, UMAX, (KC >= 16 ? 4 : 2), V, X, true, VB><<<A.lb_nblocks, kBlock, 0, s>>>(
-            row0, uoff, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
-            A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(beta));
-      else
-        k_spmm_lds<KC, UMAX, (KC >= 16 ? 4 : 2), V, X, false, VB><<<A.lb_nblocks, kBlock, 0, s>>>(
-            row0, uoff, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
-            A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(0));
-    };
-    if (vb) launch(std::true_type{});
-    else launch(std::false_type{});
+    if (beta != 0.0)
+      k_spmm_lds<KC, UMAX, (KC >= 16 ? 4 : 2), V, X, true><<<A.lb_nblocks, kBlock, 0, s>>>(
+          row0, uoff, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
+          A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(beta));
+    else
+      k_spmm_lds<KC, UMAX, (KC >= 16 ? 4 : 2), V, X, false><<<A.lb_nblocks, kBlock, 0, s>>>(
+          row0, uoff, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
+          A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(0));
   };
   // Column chunks: 8 for k <= 8 and for FP64 lists of 256, then 16 (FP64) or
   // 16 / 32 (FP32) columns; at most 16 KB of staged FP64 B, so six workgroups
@@ -966,10 +1148,14 @@ hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, con
   auto run = [&](auto vtag, auto xtag) -> hipError_t {
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
-    if (b_sc == 1 && c_sc == 1 && k >= 8 && A.lb_state == 1 && A.lb_nblocks > 0) {
+    const bool rm = b_sc == 1 && c_sc == 1;
+    if (rm && pls::spmm_on_tiles(A, dbl, k)) {
+      dispatch_tile<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
+      dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s, true);
+    } else if (rm && k >= 8 && A.lb_state == 1 && A.lb_nblocks > 0) {
       launch_lds<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
-    } else if (b_sc == 1 && c_sc == 1) {
-      dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
+    } else if (rm) {
+      dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s, false);
     } else {
       const unsigned grid = grid_for(int64_t(A.m) * k);
       if (beta != 0.0)

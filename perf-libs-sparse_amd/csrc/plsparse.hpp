@@ -99,6 +99,14 @@ struct Dense {
 };
 
 // Device CSR (0-based) with the row-block table of the adaptive kernel.
+struct LbHost;  // host form of the SpMM row blocks (spmm_blocks.cpp)
+// A tile of at most 32 rows in two halves: its first row, step and value (the
+// next tile's end them) and the rows of the first half.
+struct SpmmTile {
+  int32_t row0, step0, val0, half;
+};
+// Values past the last tile that k_spmm_tile may read ahead.
+constexpr int32_t kTilePad = 512;
 // Non-zeros of a row above which k_spmm_gather gives it a workgroup of its own
 // (power-law 1M rows, FP64 k = 8 / 64: 411 / 1702 us with 128, 387 / 1608 with
 // 256, 380 / 1577 with 512).
@@ -135,6 +143,18 @@ struct DevCsr {
   DevBuf lb_prp;         // int32 [m+1] first non-zero of each entry of the row order (clustered)
   DevBuf lb_epos;        // int32 [nnz] CSR position of each non-zero in block order (clustered)
   DevBuf lb_val;         // [nnz] vals in block order, storage vs (clustered; refreshed by updates)
+  std::shared_ptr<LbHost> lb_host;  // the cut, from which either form below is built on first use
+  bool lb_lds = false;              // the arrays above are on the device (k_spmm_lds)
+  // Row tiles of the blocks (k_spmm_tile), on the device when ntiles >= 0
+  int32_t ntiles = -1, t_ndirect = 0;
+  int64_t t_nnz = 0;  // non-zeros of the tiles
+  DevBuf t_tiles;     // SpmmTile [ntiles + 1]
+  DevBuf t_row;       // int32 rows, tile by tile
+  DevBuf t_mask;      // uint64 [2 * steps]: lanes (row + 16 * column) of each half that hold a value
+  DevBuf t_col;       // int32 [4 * steps]
+  DevBuf t_epos;      // int32 [t_nnz + kTilePad] CSR position of each value in tile order
+  DevBuf t_val;       // [t_nnz + kTilePad] values in tile order, storage vs
+  DevBuf t_direct;    // int32 [t_ndirect] rows without a list
 };
 // Limits of a column-compressed SpMM block (must match k_spmm.hip): distinct
 // columns per list (128, or 256 when lists of 128 leave too many rows without
@@ -151,6 +171,20 @@ constexpr int32_t kLbUcolsSmall = 128;
 constexpr int32_t kLbUcolsLarge = 256;
 constexpr int32_t lb_nnz_per_ucol(int32_t umax) { return umax > kLbUcolsSmall ? 8 : 7; }
 constexpr int32_t kLbRows = 128;
+
+// Whether a product with k columns runs on the row tiles (k_spmm_tile) or
+// stages the blocks' B rows in LDS (k_spmm_lds).  Tiles read a B row about as
+// often but need no barriers, and multiply on the matrix cores (27-point
+// stencil 80^3, FP64 k = 32 / 128: 168 / 555 -> 118 / 409 us, FP32 k = 64 / 128
+// 155 / 276 -> 111 / 214).  LDS stays faster for k <= 16 (half of a 32-column
+// product idle: FP64 k = 16 102 against 106 us), for short rows (5-point 500^2,
+// FP64 k = 32: 31 against 36 us: too few steps per tile) and for operands with
+// too few steps to hide a tile's latency (27-point 16^3 / 28^3, FP64 k = 32: 9 /
+// 15 against 12 / 13 us; FP32 36^3 / 45^3 12 / 21 against 14 / 21).
+inline bool spmm_on_tiles(const DevCsr &d, bool dbl, int64_t k) {
+  return d.lb_state == 1 && k > 16 && d.nnz >= 10 * int64_t(d.m) &&
+         (k > 64 || d.lb_ucols >= (dbl || k > 32 ? 100000 : 320000));
+}
 
 // Device SELL-C-sigma (layout of src/sell_c_sigma.hpp:43-104, NOTRANS).
 struct DevSell {
@@ -384,19 +418,22 @@ perflibs_status_t build_native_bsr_plan(perflibs_spmat_top_t *A);
 // The blocks of a BSR object with b = 4 or 8, uploaded for the native BSR x
 // dense product (out stays empty for any other object).
 perflibs_status_t bsr_blocks_for_spmm(perflibs_spmat_top_t *A, std::unique_ptr<DevBsr> &out);
-// Column-compressed row blocks of the wide-B SpMM kernel for the CSR plan `d`
-// of operand `o` (sets d.lb_state; a HIP error is returned as is).  rows: 0
-// keeps the cut with the shorter lists, 1 cuts consecutive rows only, 2 takes
-// the clustered cut whenever it completes.
-hipError_t build_spmm_blocks(const Operand &o, DevCsr &d, int rows = 0);
+// Column-compressed row blocks of the wide-B SpMM kernels for the CSR plan `d`
+// of operand `o`, on the host (sets d.lb_state and d.lb_host).  rows: 0 keeps
+// the cut with the shorter lists, 1 cuts consecutive rows only, 2 takes the
+// clustered cut whenever it completes.
+void build_spmm_blocks(const Operand &o, DevCsr &d, int rows = 0);
+// The device form of the blocks a product runs on (row tiles, or the blocks
+// staged in LDS), unless it is there already.
+hipError_t upload_spmm_form(const Operand &o, DevCsr &d, bool tiles);
 // The same choice on the host only, for inspection: returns 1 when the blocks
 // would be used, -1 when none gives enough reuse (the last cut tried is
 // described then); row_order[m] and block_starts[nblocks + 1] may be null.
 int spmm_blocks_host(const Operand &o, int rows, int32_t *nblocks, int32_t *list_max,
                      int64_t *list_total, int32_t *clustered, int32_t *row_order,
                      int32_t *block_starts);
-// Clustered blocks: lb_val[q] = vals[lb_epos[q]] (after the build and after
-// value updates), enqueued on the library stream.
+// Values of the device forms gathered from vals again (after value updates),
+// enqueued on the library stream.
 hipError_t refresh_block_values(DevCsr &d);
 // The device plan an SpMV with `op` runs (built on demand, src/matvec.cpp:122-129).
 perflibs_status_t ensure_plan(perflibs_spmat_top_t *A, int op);

@@ -1,6 +1,8 @@
-// spmm_blocks.cpp — row blocks of the column-compressed SpMM kernel
-// (k_spmm_lds): which rows share a workgroup, the distinct columns each block
-// lists once, and every non-zero's position in its block's list.
+// spmm_blocks.cpp — row blocks of the column-compressed SpMM kernels: which rows
+// belong together, the distinct columns each block lists once, and every
+// non-zero's position in its block's list.  Two device forms are made from the
+// cut on first use: the blocks as they are, a workgroup each (k_spmm_lds), and
+// their rows in tiles of up to 32, a wave each (k_spmm_tile).
 //
 // Two cuts are made and the one with the shorter lists kept:
 //  * consecutive: rows in order, a block closed before the row that would
@@ -23,7 +25,6 @@
 
 namespace pls {
 
-namespace {
 struct LbHost {
   std::vector<int32_t> row0{0};  // block b: entries [row0[b], row0[b+1]) of the row order
   std::vector<int32_t> uoff{0};  // block b: list entries [uoff[b], uoff[b+1]) of ucol
@@ -34,6 +35,7 @@ struct LbHost {
   int64_t cost() const { return int64_t(ucol.size()) + direct; }
 };
 
+namespace {
 template <class F> void parallel_ranges(int64_t n, int64_t min_per_range, int64_t max_ranges, F &&fn) {
   const unsigned hw = std::thread::hardware_concurrency();
   const int64_t nt =
@@ -354,7 +356,7 @@ bool cut_clustered(const Operand &o, int32_t umax, const std::vector<int32_t> &c
 // Clustered blocks also keep their non-zeros in block order: first non-zero
 // of each entry of the row order (prp), list positions, the CSR position of
 // each (epos) and the values gathered through it on the device.
-hipError_t upload_blocks(const Operand &o, const LbHost &h, int32_t umax, DevCsr &d) {
+hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
   d.lb_brow.reset();
   d.lb_prp.reset();
   d.lb_epos.reset();
@@ -400,8 +402,138 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, int32_t umax, DevCsr
       e = plk::gather_vals(d.vs, d.lb_val.get(), d.vals.get(), d.lb_epos.as<int32_t>(),
                            int64_t(nnz + 1), stream());
   }
-  d.lb_umax = umax;
-  d.lb_state = e == hipSuccess ? 1 : 0;
+  d.lb_lds = e == hipSuccess;
+  return e;
+}
+
+// Row tiles of the blocks: each block's rows in runs of at most 32, the run's
+// distinct columns four to a step, the step's values half by half in lane
+// order (row + 16 * column) behind masks of the lanes that have one.  A column
+// a row stores twice is listed twice.  Rows without a list stay outside.
+struct TileHost {
+  std::vector<SpmmTile> tiles;
+  std::vector<int32_t> row, col, epos, direct;
+  std::vector<uint64_t> mask;
+};
+hipError_t upload_tiles(const Operand &o, const LbHost &h, DevCsr &d) {
+  const int32_t base = o.prp[0];
+  const int64_t nb = int64_t(h.row0.size()) - 1;
+  std::vector<TileHost> parts(16);
+  parallel_ranges(nb, 64, 16, [&](int part, int64_t lo, int64_t hi) {
+    TileHost &P = parts[size_t(part)];
+    // list position -> tile column; tile slot (column * 32 + row) -> CSR position
+    std::vector<int32_t> pos, slot;
+    std::vector<uint8_t> halves;  // which halves of the run use a listed column
+    for (int64_t b = lo; b < hi; ++b) {
+      const int32_t r0 = h.row0[size_t(b)], nr = h.row0[size_t(b) + 1] - r0;
+      const int32_t u0 = h.uoff[size_t(b)], nu = h.uoff[size_t(b) + 1] - u0;
+      if (nu == 0 && nr == 1) {
+        const int32_t r = h.brow.empty() ? r0 : h.brow[size_t(r0)];
+        if (o.prp[r + 1] > o.prp[r]) {  // no list
+          P.direct.push_back(r);
+          continue;
+        }
+      }
+      const int32_t runs = (nr + 31) / 32;
+      for (int32_t t = 0; t < runs; ++t) {
+        const int32_t a = int32_t(int64_t(nr) * t / runs), e = int32_t(int64_t(nr) * (t + 1) / runs);
+        const int32_t half = e - a <= 16 ? e - a : (e - a + 1) / 2;
+        P.tiles.push_back({int32_t(P.row.size()), int32_t(P.mask.size() / 2), int32_t(P.epos.size()), half});
+        const size_t c0 = P.col.size();
+        // columns of the first half alone, of both, of the second alone: the
+        // steps at the ends skip a half
+        halves.assign(size_t(nu), 0);
+        for (int32_t i = a; i < e; ++i) {
+          const int32_t r = h.brow.empty() ? r0 + i : h.brow[size_t(r0 + i)];
+          P.row.push_back(r);
+          for (int32_t j = o.prp[r] - base; j < o.prp[r + 1] - base; ++j)
+            halves[h.lidx[size_t(j)]] |= i - a < half ? 1 : 2;
+        }
+        pos.assign(size_t(nu), -1);
+        for (const uint8_t cls : {1, 3, 2})
+          for (int32_t p = 0; p < nu; ++p)
+            if (halves[size_t(p)] == cls) {
+              pos[size_t(p)] = int32_t(P.col.size() - c0);
+              P.col.push_back(h.ucol[size_t(u0 + p)]);
+            }
+        slot.assign((P.col.size() - c0) * 32, -1);
+        for (int32_t i = a; i < e; ++i) {
+          const int32_t r = h.brow.empty() ? r0 + i : h.brow[size_t(r0 + i)];
+          const int32_t l = i - a < half ? i - a : 16 + i - a - half;  // half 1 from 16 on
+          for (int32_t j = o.prp[r] - base; j < o.prp[r + 1] - base; ++j) {
+            int32_t c = pos[h.lidx[size_t(j)]];
+            if (slot[size_t(c) * 32 + size_t(l)] >= 0) {  // stored twice: listed again
+              c = int32_t(P.col.size() - c0);
+              P.col.push_back(h.ucol[size_t(u0) + h.lidx[size_t(j)]]);
+              slot.resize(slot.size() + 32, -1);
+            }
+            slot[size_t(c) * 32 + size_t(l)] = j;
+          }
+        }
+        while ((P.col.size() - c0) % 4 != 0) {
+          P.col.push_back(P.col.back());
+          slot.resize(slot.size() + 32, -1);
+        }
+        for (size_t s = 0; s < slot.size(); s += 128)
+          for (int hf = 0; hf < 2; ++hf) {
+            uint64_t m = 0;
+            for (int l = 0; l < 64; ++l) {
+              const int32_t j = slot[s + size_t(l / 16) * 32 + size_t(hf * 16 + l % 16)];
+              if (j < 0) continue;
+              m |= uint64_t(1) << l;
+              P.epos.push_back(j);
+            }
+            P.mask.push_back(m);
+          }
+      }
+    }
+  });
+  size_t nt = 0, nr = 0, nc = 0, nv = 0, nd = 0;
+  for (TileHost &P : parts) {  // positions in the whole arrays
+    for (SpmmTile &t : P.tiles) {
+      t.row0 += int32_t(nr);
+      t.step0 += int32_t(nc / 4);
+      t.val0 += int32_t(nv);
+    }
+    nt += P.tiles.size();
+    nr += P.row.size();
+    nc += P.col.size();
+    nv += P.epos.size();
+    nd += P.direct.size();
+  }
+  // the kernel reads whole groups of values ahead: padding (the CSR plan's own
+  // padding value)
+  TileHost end;
+  end.tiles.push_back({int32_t(nr), int32_t(nc / 4), int32_t(nv), 0});
+  end.epos.assign(size_t(kTilePad), int32_t(int64_t(o.prp[o.m]) - base));
+  parts.push_back(std::move(end));
+  const size_t es = d.vs == VStore::F64 ? 8 : d.vs == VStore::F32 ? 4 : 2;
+  hipError_t e = hipSuccess;
+  auto put = [&](DevBuf &dst, auto member) {
+    size_t bytes = 0;
+    for (const TileHost &P : parts) bytes += (P.*member).size() * sizeof((P.*member)[0]);
+    if (e == hipSuccess) e = dst.alloc(std::max<size_t>(bytes, 8));
+    size_t at = 0;
+    for (const TileHost &P : parts) {
+      const size_t n = (P.*member).size() * sizeof((P.*member)[0]);
+      if (e == hipSuccess && n)
+        e = hipMemcpy(static_cast<char *>(dst.get()) + at, (P.*member).data(), n, hipMemcpyHostToDevice);
+      at += n;
+    }
+  };
+  put(d.t_tiles, &TileHost::tiles);
+  put(d.t_row, &TileHost::row);
+  put(d.t_mask, &TileHost::mask);
+  put(d.t_col, &TileHost::col);
+  put(d.t_epos, &TileHost::epos);
+  put(d.t_direct, &TileHost::direct);
+  if (e == hipSuccess) e = d.t_val.alloc(es * (nv + size_t(kTilePad)));
+  d.t_nnz = int64_t(nv);
+  d.t_ndirect = int32_t(nd);
+  if (e == hipSuccess)
+    e = plk::gather_vals(d.vs, d.t_val.get(), d.vals.get(), d.t_epos.as<int32_t>(),
+                         d.t_nnz + kTilePad, stream());
+  d.ntiles = e == hipSuccess ? int32_t(nt) : -1;
   return e;
 }
 }  // namespace
@@ -458,17 +590,23 @@ bool choose_blocks(const Operand &o, int rows, LbHost &out, int32_t &umax_out) {
 }
 }  // namespace
 
-hipError_t build_spmm_blocks(const Operand &o, DevCsr &d, int rows) {
-  LbHost h;
+void build_spmm_blocks(const Operand &o, DevCsr &d, int rows) {
+  auto h = std::make_shared<LbHost>();
   int32_t umax = 0;
-  const bool used = choose_blocks(o, rows, h, umax);
-  d.lb_nblocks = int32_t(h.row0.size() - 1);
-  d.lb_ucols = int64_t(h.ucol.size());
+  const bool used = choose_blocks(o, rows, *h, umax);
+  d.lb_nblocks = int32_t(h->row0.size() - 1);
+  d.lb_ucols = int64_t(h->ucol.size());
   d.lb_umax = umax;
-  d.lb_clustered = !h.brow.empty();
-  if (used) return upload_blocks(o, h, umax, d);
-  d.lb_state = -1;
-  return hipSuccess;
+  d.lb_clustered = !h->brow.empty();
+  d.lb_lds = false;
+  d.ntiles = -1;
+  d.lb_host = used ? std::move(h) : nullptr;
+  d.lb_state = used ? 1 : -1;
+}
+
+hipError_t upload_spmm_form(const Operand &o, DevCsr &d, bool tiles) {
+  if (d.lb_state != 1 || (tiles ? d.ntiles >= 0 : d.lb_lds)) return hipSuccess;
+  return tiles ? upload_tiles(o, *d.lb_host, d) : upload_blocks(o, *d.lb_host, d);
 }
 
 int spmm_blocks_host(const Operand &o, int rows, int32_t *nblocks, int32_t *list_max,
@@ -489,9 +627,15 @@ int spmm_blocks_host(const Operand &o, int rows, int32_t *nblocks, int32_t *list
 }
 
 hipError_t refresh_block_values(DevCsr &d) {
-  if (d.lb_state != 1 || !d.lb_clustered || !d.lb_val.get()) return hipSuccess;
-  return plk::gather_vals(d.vs, d.lb_val.get(), d.vals.get(), d.lb_epos.as<int32_t>(), d.nnz + 1,
-                          stream());
+  hipError_t e = hipSuccess;
+  if (d.lb_state != 1) return e;
+  if (d.lb_lds && d.lb_clustered)
+    e = plk::gather_vals(d.vs, d.lb_val.get(), d.vals.get(), d.lb_epos.as<int32_t>(), d.nnz + 1,
+                         stream());
+  if (e == hipSuccess && d.ntiles >= 0)
+    e = plk::gather_vals(d.vs, d.t_val.get(), d.vals.get(), d.t_epos.as<int32_t>(),
+                         d.t_nnz + kTilePad, stream());
+  return e;
 }
 
 }  // namespace pls
