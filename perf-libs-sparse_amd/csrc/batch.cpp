@@ -1,4 +1,4 @@
-// batch.cpp — batched uneven SpMV / SpMM in one persistent launch.
+// batch.cpp — batched uneven SpMV / SpMM in one graph launch.
 //
 // A batch holds nprob CSR products Y_p = alpha*A_p*X_p + beta*Y_p with
 // k_p in {1, 2, 4, 8, 16} right-hand sides.  HBM layout: all problems' 0-based
@@ -13,8 +13,8 @@
 // sell_structure): a chunk table, columns, values and a slot -> row map, built
 // on the host from the device copy of those problems.
 //
-// exec launches one kernel over all tiles from a hipGraph captured once per
-// (alpha, beta, shape).  optimize(autotune) times candidate tile sizes,
+// exec launches one kernel over all CSR tiles (and one over the SELL-C-sigma
+// tiles) from a hipGraph captured once per (alpha, beta, shape).  optimize(autotune) times candidate tile sizes,
 // per-k-class row shapes (lanes per row, columns per lane) and the SELL-C-sigma
 // (C, sigma) of the k = 1 problems by graph replays on scratch outputs and
 // keeps the fastest, one coordinate at a time.
@@ -44,11 +44,11 @@ struct perflibs_amd_batch_s {
   int64_t y_total = 0;
   bool has_class[kBatchClasses] = {false, false, false, false, false};
   double mean_row[kBatchClasses] = {0, 0, 0, 0, 0};
-  pls::DevBuf rp, ci, vals, probs_d, tiles_d, xs, ys;
+  pls::DevBuf rp, ci, vals, tiles_d, xs, ys;
   bool operands = false;
   int32_t tile_nnz = 2048;
   BatchShape shape{};
-  int32_t ntiles = 0, grid = 0;
+  int32_t ntiles = 0, ncsr = 0, grid = 0;
   int32_t cus = 1, occ = 1;
   // SELL-C-sigma layout of the k = 1 problems (sell_C 0: they run as CSR tiles)
   int32_t sell_C = 0, sell_sigma = 0;
@@ -98,7 +98,8 @@ perflibs_status_t batch_fail(perflibs_status_t st, const std::string &msg) {
 // Row tiles of at most tile_nnz non-zeros (a longer row is a tile of its own)
 // and at most plk::batch_staged_rows() rows (512 for FP64, 1024 for FP32
 // accumulation), so a tile of up to plk::kBatchStage non-zeros is staged in
-// LDS by the kernel; sorted by estimated bytes moved, largest first.
+// LDS by the kernel; sorted by estimated bytes moved, largest first, the CSR
+// tiles before the SELL-C-sigma ones (a launch each).
 void build_tiles(const perflibs_amd_batch_s &B, int32_t tile_nnz, std::vector<BatchTile> &tiles) {
   struct Costed {
     double cost;
@@ -124,7 +125,7 @@ void build_tiles(const perflibs_amd_batch_s &B, int32_t tile_nnz, std::vector<Ba
         }
         const double rows = double(c - c0) * B.sell_C;
         const double cost = double(slots) * (sv + 4 + sx / 4) + rows * sx * 2;
-        all.push_back({cost, BatchTile{int32_t(p), c0, c, 1}});
+        all.push_back({cost, BatchTile{int32_t(p), c0, c, 1, 0, 0, 0, 0, 0, 1, 0, 0}});
       }
       continue;
     }
@@ -141,11 +142,14 @@ void build_tiles(const perflibs_amd_batch_s &B, int32_t tile_nnz, std::vector<Ba
       }
       const double rows = r - r0;
       const double cost = double(nz) * (sv + 4 + pb.k * sx / 4) + rows * pb.k * sx * 2;
-      all.push_back({cost, BatchTile{int32_t(p), r0, r, 0}});
+      all.push_back({cost, BatchTile{int32_t(p), r0, r, 0, pb.rp_off + r0, pb.nz_off + rp[r0], rp[r0],
+                                     int32_t(nz), r - r0, pb.k, pb.kclass, 0}});
     }
   }
   std::stable_sort(all.begin(), all.end(),
-                   [](const Costed &a, const Costed &b) { return a.cost > b.cost; });
+                   [](const Costed &a, const Costed &b) {
+                     return a.t.kind != b.t.kind ? a.t.kind < b.t.kind : a.cost > b.cost;
+                   });
   tiles.resize(all.size());
   for (size_t i = 0; i < all.size(); ++i) tiles[i] = all[i].t;
 }
@@ -154,6 +158,7 @@ perflibs_status_t upload_tiles(perflibs_amd_batch_s *B) {
   std::vector<BatchTile> tiles;
   build_tiles(*B, B->tile_nnz, tiles);
   B->ntiles = int32_t(tiles.size());
+  B->ncsr = int32_t(std::count_if(tiles.begin(), tiles.end(), [](const BatchTile &t) { return t.kind == 0; }));
   B->grid = int32_t(std::min<int64_t>(B->ntiles, int64_t(B->cus) * B->occ));
   hipError_t e = hipStreamSynchronize(stream());
   if (e == hipSuccess) e = B->tiles_d.upload(tiles.data(), sizeof(BatchTile) * std::max<size_t>(tiles.size(), 1));
@@ -168,9 +173,9 @@ plk::BatchLaunch launch_of(const perflibs_amd_batch_s *B, const void *xs, const 
   L.dbl = B->dt == DType::F64;
   L.vs = B->vs;
   L.ntiles = B->ntiles;
+  L.ncsr = B->ncsr;
   L.grid = B->grid;
   L.tiles = B->tiles_d.as<BatchTile>();
-  L.probs = B->probs_d.as<BatchProblem>();
   L.rp = B->rp.as<int32_t>();
   L.ci = B->ci.as<int32_t>();
   L.vals = B->vals.get();
@@ -444,8 +449,6 @@ perflibs_status_t perflibs_amd_batch_create(perflibs_amd_batch_t *out, int64_t n
       if (e == hipSuccess) e = hipStreamSynchronize(stream());
     }
   }
-  if (e == hipSuccess)
-    e = B->probs_d.upload(B->probs.data(), sizeof(BatchProblem) * std::max<size_t>(B->probs.size(), 1));
   if (e == hipSuccess) e = B->xs.alloc(sizeof(void *) * size_t(std::max<int64_t>(nprob, 1)));
   if (e == hipSuccess) e = B->ys.alloc(sizeof(void *) * size_t(std::max<int64_t>(nprob, 1)));
   if (e != hipSuccess) return batch_fail(PERFLIBS_STATUS_EXECUTION_FAILURE, "batch upload failed");

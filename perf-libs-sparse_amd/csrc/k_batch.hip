@@ -1,4 +1,4 @@
-// k_batch.hip — one persistent launch over a batch of independent CSR
+// k_batch.hip — a persistent launch over a batch of independent CSR
 // products Y_p = alpha * A_p * X_p + beta * Y_p (X_p: n_p x k_p, Y_p: m_p x k_p,
 // row-major; k_p = 1 is SpMV).
 //
@@ -14,6 +14,9 @@
 // the batch autotuner.  Same per-row arithmetic as the single-matrix CSR
 // kernels (src/compressed_sparse_rows.cpp:1114-1138 for k = 1 and the
 // row-blocked SpMM, src/compressed_sparse_rows.cpp:1699-1763, for k > 1).
+#include <algorithm>
+#include <type_traits>
+
 #include "k_batch.hpp"
 #include "k_common.hpp"
 
@@ -31,72 +34,97 @@ template <class A> struct BatchLds {
   int32_t rp[kBatchRows<A> + 1];
 };
 
-template <int CPL, class V, class X, bool BETA>
-__device__ __forceinline__ void batch_tile(const BatchTile &tl, const BatchProblem &pb, int G,
+// A tile on its way into LDS: a thread's entry pairs and row offsets.
+template <class A> struct BatchRegs {
+  static constexpr int NP = kBatchStage / kBlock / 2;
+  static constexpr int NR = kBatchRows<A> / kBlock + 1;
+  int32_t c[NP][2];
+  A a[NP][2];
+  int32_t r[NR];
+};
+
+template <class A> __device__ __forceinline__ bool batch_staged(const BatchTile &tl) {
+  return tl.nnz <= kBatchStage && tl.nrows <= kBatchRows<A>;
+}
+
+// Loads a staged tile's entries in pairs (one 8-byte index load, one 2-value
+// load) from the even index at or below its first; the batch arrays end with
+// one padding entry, so the last pair stays in bounds.
+template <class V, class A>
+__device__ __forceinline__ void batch_load(const BatchTile &tl, const int32_t *__restrict__ rp_all,
+                                           const int32_t *__restrict__ ci_all,
+                                           const V *__restrict__ val_all, BatchRegs<A> &g) {
+  const int tid = threadIdx.x;
+  if (!batch_staged<A>(tl)) return;
+  const int32_t *rp = rp_all + tl.rp0;
+#pragma unroll
+  for (int u = 0; u < BatchRegs<A>::NR; ++u) g.r[u] = rp[min(tid + u * kBlock, tl.nrows)];
+  if (tl.nnz == 0) return;
+  const int32_t sh = int32_t(tl.nz0 & 1);
+  const int32_t *cia = ci_all + (tl.nz0 - sh);
+  const V *vaa = val_all + (tl.nz0 - sh);
+  const int32_t lastp = (tl.nnz + sh - 1) & ~1;  // last pair holding a tile entry
+#pragma unroll
+  for (int u = 0; u < BatchRegs<A>::NP; ++u)
+    ld_pair(cia, vaa, min(2 * (tid + u * kBlock), lastp), g.c[u], g.a[u]);
+}
+
+template <class V, class A>
+__device__ __forceinline__ void batch_store(const BatchTile &tl, const int32_t *__restrict__ ci_all,
+                                            const V *__restrict__ val_all, A alpha,
+                                            const BatchRegs<A> &g, BatchLds<A> &lds) {
+  const int tid = threadIdx.x;
+  if (!batch_staged<A>(tl)) return;
+#pragma unroll
+  for (int u = 0; u < BatchRegs<A>::NR; ++u)
+    if (tid + u * kBlock <= tl.nrows) lds.rp[tid + u * kBlock] = g.r[u] - tl.e0;
+  const int32_t sh = int32_t(tl.nz0 & 1);
+#pragma unroll
+  for (int u = 0; u < BatchRegs<A>::NP; ++u) {
+    const int32_t q = 2 * (tid + u * kBlock) - sh;  // tile position of the pair's first entry
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (q + h >= 0 && q + h < tl.nnz) {
+        lds.ci[q + h] = g.c[u][h];
+        lds.a[q + h] = alpha * g.a[u][h];
+      }
+  }
+  // a full tile from an odd index has one entry past the pairs
+  if (sh && tid == 0 && tl.nnz == kBatchStage) {
+    lds.ci[tl.nnz - 1] = ldi(ci_all, tl.nz0 + tl.nnz - 1);
+    lds.a[tl.nnz - 1] = alpha * A(ldv(val_all, tl.nz0 + tl.nnz - 1));
+  }
+}
+
+template <int CPL, bool STAGED, class V, class X, bool BETA>
+__device__ __forceinline__ void batch_rows(const BatchTile &tl, int G,
                                            const int32_t *__restrict__ rp_all,
                                            const int32_t *__restrict__ ci_all,
                                            const V *__restrict__ val_all,
                                            const X *__restrict__ xp, X *__restrict__ yp,
                                            acc_t<X> alpha, acc_t<X> beta,
-                                           BatchLds<acc_t<X>> &lds) {
+                                           const BatchLds<acc_t<X>> &lds) {
   using A = acc_t<X>;
-  const int k = pb.k;
+  typedef X XV __attribute__((ext_vector_type(CPL), aligned(sizeof(X))));
+  const int k = tl.k;
   const int kc = k / CPL;  // lanes spanning one row's k columns
   const int S = G / kc;    // non-zero subsets per row
-  const int32_t *rp = rp_all + pb.rp_off;
-  const int32_t *ci = ci_all + pb.nz_off;
-  const V *va = val_all + pb.nz_off;
+  const int32_t *rp = rp_all + tl.rp0;
+  const int32_t *ci = ci_all + tl.nz0;
+  const V *va = val_all + tl.nz0;
   const int tid = threadIdx.x;
   const int lane = tid & (G - 1), grp = tid / G;
   const int sub = lane / kc, cb = (lane % kc) * CPL;
   const int rows_per_pass = kBlock / G;
   const bool products = alpha != A(0);
-  const int32_t e0 = rp[tl.r0];
-  const int32_t nnz = rp[tl.r1] - e0, nrows = tl.r1 - tl.r0;
-  const bool staged = nnz <= kBatchStage && nrows <= kBatchRows<A>;
-  __syncthreads();  // the previous tile is done with the LDS
-  if (staged) {
-    if (nnz > 0) {
-      // entry pairs (one 8-byte index load, one 2-value load) from the even
-      // absolute index at or below the tile's first entry; the batch arrays
-      // end with one padding entry, so the last pair stays in bounds
-      constexpr int NP = kBatchStage / kBlock / 2;
-      const int64_t g0 = int64_t(pb.nz_off) + e0;
-      const int32_t sh = int32_t(g0 & 1);
-      const int32_t *cia = ci_all + (g0 - sh);
-      const V *vaa = val_all + (g0 - sh);
-      const int32_t lastp = (nnz + sh - 1) & ~1;  // last pair holding a tile entry
-      int32_t c[NP][2];
-      A a[NP][2];
-#pragma unroll
-      for (int u = 0; u < NP; ++u) ld_pair(cia, vaa, min(2 * (tid + u * kBlock), lastp), c[u], a[u]);
-#pragma unroll
-      for (int u = 0; u < NP; ++u) {
-        const int32_t q = 2 * (tid + u * kBlock) - sh;  // tile position of the pair's first entry
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          if (q + h >= 0 && q + h < nnz) {
-            lds.ci[q + h] = c[u][h];
-            lds.a[q + h] = alpha * a[u][h];
-          }
-      }
-      // a full tile from an odd index has one entry past the pairs
-      if (sh && tid == 0 && nnz == kBatchStage) {
-        lds.ci[nnz - 1] = ldi(ci, e0 + nnz - 1);
-        lds.a[nnz - 1] = alpha * A(ldv(va, e0 + nnz - 1));
-      }
-    }
-    for (int32_t q = tid; q <= nrows; q += kBlock) lds.rp[q] = rp[tl.r0 + q] - e0;
-  }
-  __syncthreads();
-  for (int32_t base = 0; base < nrows; base += rows_per_pass) {
+  for (int32_t base = 0; base < tl.nrows; base += rows_per_pass) {
     const int32_t rr = base + grp;
     A acc[CPL];
 #pragma unroll
     for (int t = 0; t < CPL; ++t) acc[t] = A(0);
-    if (rr < nrows && products) {
-      const int32_t p0 = staged ? lds.rp[rr] : rp[tl.r0 + rr] - e0;
-      const int32_t p1 = staged ? lds.rp[rr + 1] : rp[tl.r0 + rr + 1] - e0;
+    if (rr < tl.nrows && products) {
+      const int32_t p0 = STAGED ? lds.rp[rr] : rp[rr] - tl.e0;
+      const int32_t p1 = STAGED ? lds.rp[rr + 1] : rp[rr + 1] - tl.e0;
       constexpr int U = CPL >= 4 ? 4 : 8;  // non-zeros in flight per lane
       for (int32_t j = p0 + sub; j < p1; j += U * S) {
         int32_t c[U];
@@ -104,32 +132,35 @@ __device__ __forceinline__ void batch_tile(const BatchTile &tl, const BatchProbl
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int32_t jj = min(j + u * S, p1 - 1);
-          c[u] = staged ? lds.ci[jj] : ldi(ci, e0 + jj);
-          a[u] = staged ? lds.a[jj] : alpha * A(ldv(va, e0 + jj));
+          c[u] = STAGED ? lds.ci[jj] : ldi(ci, jj);
+          a[u] = STAGED ? lds.a[jj] : alpha * A(ldv(va, jj));
         }
+        XV x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          x[u] = *reinterpret_cast<const XV *>(xp + int64_t(c[u]) * k + cb);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const X *xr = xp + int64_t(c[u]) * k + cb;
           const bool ok = j + u * S < p1;
 #pragma unroll
-          for (int t = 0; t < CPL; ++t) {
-            const A p = a[u] * A(xr[t]);
-            acc[t] += ok ? p : A(0);
-          }
+          for (int t = 0; t < CPL; ++t) acc[t] = ok ? acc[t] + a[u] * A(x[u][t]) : acc[t];
         }
       }
     }
     for (int o = kc; o < G; o <<= 1)
 #pragma unroll
       for (int t = 0; t < CPL; ++t) acc[t] += __shfl_xor(acc[t], o);
-    if (rr < nrows && sub == 0) {
-      X *yr = yp + int64_t(tl.r0 + rr) * k + cb;
+    if (rr < tl.nrows && sub == 0) {
+      XV *yr = reinterpret_cast<XV *>(yp + int64_t(tl.r0 + rr) * k + cb);
+      XV o;
+      if (BETA) o = *yr;
 #pragma unroll
       for (int t = 0; t < CPL; ++t) {
         A r = acc[t];
-        if (BETA) r += beta * A(yr[t]);
-        yr[t] = X(r);
+        if (BETA) r += beta * A(o[t]);
+        o[t] = X(r);
       }
+      *yr = o;
     }
   }
 }
@@ -139,19 +170,20 @@ __device__ __forceinline__ void batch_tile(const BatchTile &tl, const BatchProbl
 // column / value slices of a chunk are contiguous across its lanes, so each
 // step of the row loop is one coalesced load per array; padding slots hold
 // value 0 and column 0 of the problem.  Four non-zeros in flight per lane.
-// Kept out of line: inlined into k_batch it changed the register allocation of
-// the CSR tile loop and made the CSR tiles 1.6x slower (FP32 batch 4.77 ->
-// 7.52 ms, FP64 7.89 -> 12.71 ms at the same shape); as a call it costs the
-// CSR tiles nothing.
+// A kernel of its own, launched after the CSR tiles': it needs no LDS and a
+// quarter of their registers (256 banded problems, all k = 1, C = 32: FP64 /
+// FP32 379 / 297 us as tiles of one kernel, 261 / 192 on its own; the two
+// launches as parallel branches of the graph took 615 us where one after the
+// other take 496).
 template <int C, class V, class X, bool BETA>
-__device__ __noinline__ void batch_sell_tile(const BatchTile &tl,
-                                                const BatchSellChunk *__restrict__ chunks,
-                                                const int32_t *__restrict__ sci,
-                                                const V *__restrict__ sval,
-                                                const int32_t *__restrict__ perm,
-                                                const X *__restrict__ xp, X *__restrict__ yp,
-                                                acc_t<X> alpha, acc_t<X> beta) {
+__global__ __launch_bounds__(kBlock) void k_batch_sell(
+    const BatchTile *__restrict__ tiles, const BatchSellChunk *__restrict__ chunks,
+    const int32_t *__restrict__ sci, const V *__restrict__ sval, const int32_t *__restrict__ perm,
+    const X *const *__restrict__ xs, X *const *__restrict__ ys, acc_t<X> alpha, acc_t<X> beta) {
   using A = acc_t<X>;
+  const BatchTile tl = tiles[blockIdx.x];
+  const X *xp = xs[tl.prob];
+  X *yp = ys[tl.prob];
   const int tid = threadIdx.x, r = tid % C;
   for (int32_t c = tl.r0 + tid / C; c < tl.r1; c += kBlock / C) {
     const BatchSellChunk ch = chunks[c];
@@ -182,38 +214,52 @@ __device__ __noinline__ void batch_sell_tile(const BatchTile &tl,
   }
 }
 
+// A workgroup has its next tile's record, entries and row offsets on their way
+// (in registers) while it computes the current one from LDS: a tile then waits
+// for its X rows only (256 banded problems, FP64 / FP32: 508 / 317 -> 495 / 295
+// us).  That takes 125 VGPRs in FP64, so four workgroups share a CU; five or six
+// spill and take 792 / 952 us.
 template <class V, class X, bool BETA>
-// At least six waves per SIMD: caps the FP64 kernel at 84 VGPRs (86 without),
-// which with 26 KB of LDS lets six workgroups share a CU (FP64 batch 7.93 ->
-// 7.75 ms); the FP32 kernels use fewer registers anyway.
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_batch(
-    int32_t ntiles, const BatchTile *__restrict__ tiles, const BatchProblem *__restrict__ probs,
-    const int32_t *__restrict__ rp_all, const int32_t *__restrict__ ci_all,
-    const V *__restrict__ val_all, const X *const *__restrict__ xs, X *const *__restrict__ ys,
-    acc_t<X> alpha, acc_t<X> beta, BatchShape shape, int32_t sell_C,
-    const BatchSellChunk *__restrict__ chunks, const int32_t *__restrict__ sci,
-    const V *__restrict__ sval, const int32_t *__restrict__ perm) {
-  __shared__ BatchLds<acc_t<X>> lds;
-  for (int32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const BatchTile tl = tiles[t];
-    const X *xp = xs[tl.prob];
-    X *yp = ys[tl.prob];
-    if (tl.kind == 1) {  // no LDS: the next CSR tile's barrier does not wait on it
-      if (sell_C == 32)
-        batch_sell_tile<32, V, X, BETA>(tl, chunks, sci, sval, perm, xp, yp, alpha, beta);
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_batch(
+    int32_t ntiles, const BatchTile *__restrict__ tiles, const int32_t *__restrict__ rp_all,
+    const int32_t *__restrict__ ci_all, const V *__restrict__ val_all,
+    const X *const *__restrict__ xs, X *const *__restrict__ ys, acc_t<X> alpha, acc_t<X> beta,
+    BatchShape shape) {
+  using A = acc_t<X>;
+  __shared__ BatchLds<A> lds;
+  BatchRegs<A> g;
+  int32_t t = blockIdx.x;
+  if (t >= ntiles) return;
+  BatchTile tl = tiles[t];
+  const X *xp = xs[tl.prob];
+  X *yp = ys[tl.prob];
+  batch_load(tl, rp_all, ci_all, val_all, g);
+  for (;;) {
+    const int32_t nt = t + gridDim.x;
+    const bool more = nt < ntiles;
+    BatchTile next = tl;
+    if (more) next = tiles[nt];
+    __syncthreads();  // the previous tile is done with the LDS
+    batch_store(tl, ci_all, val_all, alpha, g, lds);
+    if (more) batch_load(next, rp_all, ci_all, val_all, g);
+    __syncthreads();
+    const int G = shape.lanes[tl.kclass];
+    const int cpl = shape.cpl[tl.kclass];
+    auto rows = [&](auto ctag) {
+      constexpr int CPL = decltype(ctag)::value;
+      if (batch_staged<A>(tl))
+        batch_rows<CPL, true, V, X, BETA>(tl, G, rp_all, ci_all, val_all, xp, yp, alpha, beta, lds);
       else
-        batch_sell_tile<64, V, X, BETA>(tl, chunks, sci, sval, perm, xp, yp, alpha, beta);
-      continue;
-    }
-    const BatchProblem pb = probs[tl.prob];
-    const int G = shape.lanes[pb.kclass];
-    const int cpl = shape.cpl[pb.kclass];
-    if (cpl == 1)
-      batch_tile<1, V, X, BETA>(tl, pb, G, rp_all, ci_all, val_all, xp, yp, alpha, beta, lds);
-    else if (cpl == 2)
-      batch_tile<2, V, X, BETA>(tl, pb, G, rp_all, ci_all, val_all, xp, yp, alpha, beta, lds);
-    else
-      batch_tile<4, V, X, BETA>(tl, pb, G, rp_all, ci_all, val_all, xp, yp, alpha, beta, lds);
+        batch_rows<CPL, false, V, X, BETA>(tl, G, rp_all, ci_all, val_all, xp, yp, alpha, beta, lds);
+    };
+    if (cpl == 1) rows(std::integral_constant<int, 1>{});
+    else if (cpl == 2) rows(std::integral_constant<int, 2>{});
+    else rows(std::integral_constant<int, 4>{});
+    if (!more) return;
+    tl = next;
+    t = nt;
+    xp = xs[tl.prob];
+    yp = ys[tl.prob];
   }
 }
 
@@ -237,14 +283,22 @@ hipError_t batch_launch(const BatchLaunch &L, hipStream_t s) {
     const auto *xs = static_cast<const X *const *>(L.xs);
     auto *ys = static_cast<X *const *>(L.ys);
     const auto *sv = static_cast<const V *>(L.svals);
-    if (L.beta != 0.0)
-      k_batch<V, X, true><<<L.grid, kBlock, 0, s>>>(
-          L.ntiles, L.tiles, L.probs, L.rp, L.ci, static_cast<const V *>(L.vals), xs, ys,
-          acc_t<X>(L.alpha), acc_t<X>(L.beta), L.shape, L.sell_C, L.chunks, L.sci, sv, L.perm);
-    else
-      k_batch<V, X, false><<<L.grid, kBlock, 0, s>>>(
-          L.ntiles, L.tiles, L.probs, L.rp, L.ci, static_cast<const V *>(L.vals), xs, ys,
-          acc_t<X>(L.alpha), acc_t<X>(0), L.shape, L.sell_C, L.chunks, L.sci, sv, L.perm);
+    const auto *tiles = L.tiles;
+    auto csr = [&](auto kern) {
+      kern<<<std::min(L.grid, L.ncsr), kBlock, 0, s>>>(
+          L.ncsr, tiles, L.rp, L.ci, static_cast<const V *>(L.vals), xs, ys, acc_t<X>(L.alpha),
+          acc_t<X>(L.beta), L.shape);
+    };
+    auto sell = [&](auto kern) {
+      kern<<<L.ntiles - L.ncsr, kBlock, 0, s>>>(tiles + L.ncsr, L.chunks, L.sci, sv, L.perm, xs, ys,
+                                                acc_t<X>(L.alpha), acc_t<X>(L.beta));
+    };
+    const bool upd = L.beta != 0.0;
+    if (L.ncsr > 0) upd ? csr(k_batch<V, X, true>) : csr(k_batch<V, X, false>);
+    if (L.ntiles > L.ncsr) {
+      if (L.sell_C == 32) upd ? sell(k_batch_sell<32, V, X, true>) : sell(k_batch_sell<32, V, X, false>);
+      else upd ? sell(k_batch_sell<64, V, X, true>) : sell(k_batch_sell<64, V, X, false>);
+    }
     return hipGetLastError();
   });
 }
@@ -254,8 +308,8 @@ int batch_occupancy(bool dbl, pls::VStore vs) {
   hipError_t e = batch_types(vs, dbl, [&](auto vtag, auto xtag) -> hipError_t {
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &nb, reinterpret_cast<const void *>(&k_batch<V, X, false>), kBlock, 0);
+    const void *kern = reinterpret_cast<const void *>(&k_batch<V, X, false>);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, kBlock, 0);
   });
   return e == hipSuccess ? nb : 0;
 }

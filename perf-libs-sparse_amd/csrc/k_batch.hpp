@@ -28,9 +28,14 @@ struct BatchProblem {
 };
 
 // kind 0: rows [r0, r1) of problem `prob` (CSR); kind 1: SELL-C-sigma chunks
-// [r0, r1) of the batch's chunk table, all of problem `prob` (k = 1 only).
+// [r0, r1) of the batch's chunk table, all of problem `prob` (k = 1 only).  A
+// CSR tile's record holds all the kernel needs to load it: where its row
+// pointers and non-zeros start in the batch arrays, its first row pointer's
+// value e0, sizes, k and k class.
 struct BatchTile {
   int32_t prob, r0, r1, kind;
+  int64_t rp0, nz0;
+  int32_t e0, nnz, nrows, k, kclass, pad;
 };
 
 // A SELL-C-sigma chunk of a k = 1 problem (src/sell_c_sigma.cpp:145-336 layout
@@ -53,9 +58,8 @@ struct BatchShape {
 struct BatchLaunch {
   bool dbl = true;
   pls::VStore vs = pls::VStore::F64;
-  int32_t ntiles = 0, grid = 0;
+  int32_t ntiles = 0, ncsr = 0, grid = 0;  // the first ncsr tiles are CSR, the rest SELL-C-sigma
   const BatchTile *tiles = nullptr;
-  const BatchProblem *probs = nullptr;
   const int32_t *rp = nullptr, *ci = nullptr;
   const void *vals = nullptr;
   const void *xs = nullptr;  // device array of nprob X pointers
