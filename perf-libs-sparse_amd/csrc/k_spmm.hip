@@ -328,22 +328,34 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
 
 // Column-compressed row blocks (k >= 8 when the plan's block lists are short
 // enough, see build_spmm_blocks, and the product is not one for the row tiles
-// above): one workgroup per block of
-// rows, consecutive ones or (brow != nullptr) the rows brow lists for the
-// block, whose non-zeros the plan keeps in block order (prp, lval, lidx: one
-// contiguous range per block, like consecutive rows).  The block's
-// alpha-scaled values and one-byte list positions are staged in LDS once (in
-// aligned pairs); then, KC columns at a time, every B row the block needs is
-// loaded into LDS once (coalesced, KC contiguous elements per row, 16 bytes per
-// lane) and each row of C is accumulated from LDS by a group of
-// KC / CPL lanes (CPL adjacent columns each, written as one vector),
-// 8 non-zeros in flight per lane.  On the 27-point stencil a staged B row
-// feeds about 5 non-zeros of a block of clustered rows (2.6 with consecutive
-// rows), so L2 -> CU traffic for B falls by that factor against the direct
-// kernels, which fetch a B row per non-zero.  A block without a list (one row
-// with more than UMAX distinct columns or lb_nnz_per_ucol(UMAX) * UMAX
-// non-zeros) spreads its non-zeros over the workgroup's lane groups, reads B
-// directly and sums the groups through LDS.
+// above): one workgroup per block of rows, consecutive ones or (brow !=
+// nullptr) the rows brow lists for the block, whose non-zeros the plan keeps in
+// block order (prp, lval, lidx: one contiguous range per block, like
+// consecutive rows).  The block's alpha-scaled values and list positions are
+// staged in LDS once (loaded in aligned pairs); then, KC columns at a time,
+// every B row the block needs is loaded into LDS once (coalesced, KC contiguous
+// elements per row, 16 bytes per lane) and each row of C is accumulated from
+// LDS by a group of KC / CPL lanes (CPL adjacent columns each, written as one
+// vector), 8 non-zeros in flight per lane.  On the 27-point stencil a staged B
+// row feeds about 5 non-zeros of a block of clustered rows (2.6 with
+// consecutive rows), so L2 -> CU traffic for B falls by that factor against the
+// direct kernels, which fetch a B row per non-zero.
+// Bound by the block's chain of loads and barriers and by the instructions per
+// non-zero (FP32, k = 8: vector units busy 70% of the time when every step of 8
+// masked its tail).  So a row is walked in steps of 8, 4, 2 and 1 without masks
+// (from 4 where a lane's columns take more than 16 bytes: the registers of 8
+// cost FP64 k = 16 a workgroup per CU, 98 -> 109 us), and FP32 chunks of up to
+// 16 columns keep an entry as one 8-byte LDS read, value and byte offset of its
+// B row (PACK; chunks of 32 lose a workgroup by the larger entries, 5-point 80^3
+// k = 32 47.4 -> 49.3 us).  Masked steps of 8 -> now, us: 27-point 80^3 FP32 k =
+// 8 / 16 59.1 / 66.7 -> 54.6 / 60.0, FP64 68.0 / 100.1 -> 64.9 / 97.7; 5-point
+// 1000^2 FP32 k = 8 / 32 34.2 / 66.2 -> 32.0 / 63.3; 8 x 8 block stencil FP64 k =
+// 16 50.1 -> 42.8.  A row's parts summed in contiguous pieces or four columns
+// per lane at k = 8 is slower (FP64 77 us), as is a persistent launch that
+// prefetches the next block: it loses its occupancy (FP32 k = 8 / 16 61 / 83).
+// A block without a list (one row with more than UMAX distinct columns or
+// lb_nnz_per_ucol(UMAX) * UMAX non-zeros) spreads its non-zeros over the
+// workgroup's lane groups, reads B directly and sums the groups through LDS.
 template <int KC, int UMAX, int CPL, class V, class X, bool BETA>
 __global__ __launch_bounds__(kBlock) void k_spmm_lds(
     const int32_t *__restrict__ row0s, const int32_t *__restrict__ uoff,
@@ -355,8 +367,11 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
   using A = acc_t<X>;
   constexpr int NG = kBlock / KC;  // lane groups (rows in flight) per workgroup
   __shared__ __align__(16) A sB[UMAX * KC];
-  __shared__ A s_a[pls::lb_nnz_per_ucol(UMAX) * UMAX];
-  __shared__ uint8_t s_l[pls::lb_nnz_per_ucol(UMAX) * UMAX];
+  constexpr int NNZ = pls::lb_nnz_per_ucol(UMAX) * UMAX;
+  constexpr bool PACK = KC <= 16 && sizeof(A) == 4;
+  __shared__ uint2 s_e[PACK ? NNZ : 1];  // an entry's value and byte offset of its B row
+  __shared__ A s_a[PACK ? 1 : NNZ];
+  __shared__ uint8_t s_l[PACK ? 1 : NNZ];
   __shared__ int32_t s_rp[pls::kLbRows + 1];
   __shared__ int32_t s_uc[UMAX];
   __shared__ int32_t s_row[pls::kLbRows];  // clustered blocks: the rows' indices
@@ -403,14 +418,16 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
       ld_val_pair(bval, j, v);
       const L2 l = *reinterpret_cast<const L2 *>(lidx + j);
       const int32_t q = 2 * t - sh;
-      if (q >= 0) {
-        s_a[q] = alpha * v[0];
-        s_l[q] = l.x;
-      }
-      if (q + 1 < nnz) {
-        s_a[q + 1] = alpha * v[1];
-        s_l[q + 1] = l.y;
-      }
+      auto put = [&](int32_t at, A a, uint8_t pos) {
+        if constexpr (PACK) {
+          s_e[at] = make_uint2(__float_as_uint(alpha * a), pos * uint32_t(KC * sizeof(A)));
+        } else {
+          s_a[at] = alpha * a;
+          s_l[at] = pos;
+        }
+      };
+      if (q >= 0) put(q, v[0], l.x);
+      if (q + 1 < nnz) put(q + 1, v[1], l.y);
     }
   }
   for (int32_t q = tid; q <= nrows; q += kBlock) {
@@ -462,30 +479,57 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
       A acc[CPL];
 #pragma unroll
       for (int t = 0; t < CPL; ++t) acc[t] = 0;
-      for (int32_t p = p0 + sub; p < p1; p += 8 * S) {
-        A a[8];
-        int32_t l[8];
+      if constexpr (PACK) {
+        // 8, 4, 2 and 1 entries at a time: no clamped index and no select
+        const char *bl = reinterpret_cast<const char *>(&sB[lc * CPL]);
+        auto run = [&](int32_t p, auto n) {
+          constexpr int N = decltype(n)::value;
+          typedef A XC __attribute__((ext_vector_type(CPL)));
+          uint2 e[N];
+          XC x[N];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int32_t pp = min(p + u * S, p1 - 1);
-          a[u] = p + u * S < p1 ? s_a[pp] : A(0);
-          l[u] = s_l[pp];
-        }
+          for (int u = 0; u < N; ++u) e[u] = s_e[p + u * S];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const A *b = &sB[l[u] * KC + lc * CPL];
-          if constexpr (CPL >= 2) {
-            using A2 = std::conditional_t<sizeof(A) == 8, double2, float2>;
+          for (int u = 0; u < N; ++u) x[u] = *reinterpret_cast<const XC *>(bl + e[u].y);
+#pragma unroll
+          for (int u = 0; u < N; ++u)
+#pragma unroll
+            for (int t = 0; t < CPL; ++t) acc[t] += __uint_as_float(e[u].x) * x[u][t];
+          return p + N * S;
+        };
+        int32_t p = p0 + sub;
+        while (p + 7 * S < p1) p = run(p, std::integral_constant<int, 8>{});
+        if (p + 3 * S < p1) p = run(p, std::integral_constant<int, 4>{});
+        if (p + S < p1) p = run(p, std::integral_constant<int, 2>{});
+        if (p < p1) run(p, std::integral_constant<int, 1>{});
+      } else {
+        auto run = [&](int32_t p, auto n) {
+          constexpr int N = decltype(n)::value;
+          using A2 = std::conditional_t<sizeof(A) == 8, double2, float2>;
+          A a[N];
+          int32_t l[N];
+#pragma unroll
+          for (int u = 0; u < N; ++u) a[u] = s_a[p + u * S];
+#pragma unroll
+          for (int u = 0; u < N; ++u) l[u] = s_l[p + u * S];
+#pragma unroll
+          for (int u = 0; u < N; ++u) {
+            const A *b = &sB[l[u] * KC + lc * CPL];
 #pragma unroll
             for (int h = 0; h < CPL / 2; ++h) {
               const A2 v = reinterpret_cast<const A2 *>(b)[h];
               acc[2 * h] += a[u] * v.x;
               acc[2 * h + 1] += a[u] * v.y;
             }
-          } else {
-            acc[0] += a[u] * b[0];
           }
-        }
+          return p + N * S;
+        };
+        int32_t p = p0 + sub;
+        if constexpr (CPL * sizeof(A) <= 16)
+          while (p + 7 * S < p1) p = run(p, std::integral_constant<int, 8>{});
+        while (p + 3 * S < p1) p = run(p, std::integral_constant<int, 4>{});
+        if (p + S < p1) p = run(p, std::integral_constant<int, 2>{});
+        if (p < p1) run(p, std::integral_constant<int, 1>{});
       }
 #pragma unroll
       for (int t = 0; t < CPL; ++t)
