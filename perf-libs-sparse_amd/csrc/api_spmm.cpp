@@ -160,7 +160,14 @@ perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k) {
   pls::DevCsr &d = *A->plan.csr;
   if (k < 8 || d.lb_state < 0) return PERFLIBS_STATUS_SUCCESS;
   auto tiles = [&] { return pls::spmm_on_tiles(d, A->dt == DType::F64, k); };
+  // one thread builds a form; a product on the other form does not touch it
+  const std::lock_guard<std::mutex> lock(d.lb_mutex);
   if (d.lb_state == 0 || (tiles() ? d.ntiles < 0 : !d.lb_lds)) {
+    // no allocation or copy inside a capture: csr_spmm takes the form that is there
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (d.lb_state == 1 && (d.ntiles >= 0 || d.lb_lds) &&
+        hipStreamIsCapturing(pls::stream(), &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+      return PERFLIBS_STATUS_SUCCESS;
     if (!o.prp && !pls::make_operand(A, op, o))
       return pls::exec_fail(A, "matrix format has no GPU SpMM path");
     if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);

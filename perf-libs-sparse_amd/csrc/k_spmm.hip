@@ -1193,10 +1193,10 @@ hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, con
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
     const bool rm = b_sc == 1 && c_sc == 1;
-    if (rm && pls::spmm_on_tiles(A, dbl, k)) {
+    if (rm && pls::spmm_on_tiles(A, dbl, k) && A.ntiles >= 0) {
       dispatch_tile<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
       dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s, true);
-    } else if (rm && k >= 8 && A.lb_state == 1 && A.lb_nblocks > 0) {
+    } else if (rm && k >= 8 && A.lb_lds && A.lb_nblocks > 0) {
       launch_lds<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
     } else if (rm) {
       dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s, false);

@@ -13,6 +13,7 @@
 
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -145,6 +146,7 @@ struct DevCsr {
   DevBuf lb_val;         // [nnz] vals in block order, storage vs (clustered; refreshed by updates)
   std::shared_ptr<LbHost> lb_host;  // the cut, from which either form below is built on first use
   bool lb_lds = false;              // the arrays above are on the device (k_spmm_lds)
+  std::mutex lb_mutex;              // held while a form is built
   // Row tiles of the blocks (k_spmm_tile), on the device when ntiles >= 0
   int32_t ntiles = -1, t_ndirect = 0;
   int64_t t_nnz = 0;  // non-zeros of the tiles
@@ -177,7 +179,7 @@ constexpr int32_t kLbRows = 128;
 // often but need no barriers, and multiply on the matrix cores (27-point
 // stencil 80^3, FP64 k = 32 / 128: 168 / 555 -> 118 / 409 us, FP32 k = 64 / 128
 // 155 / 276 -> 111 / 214).  LDS stays faster for k <= 16 (half of a 32-column
-// product idle: FP64 k = 16 102 against 106 us), for short rows (5-point 500^2,
+// product idle: FP64 k = 16 98 against 106 us), for short rows (5-point 500^2,
 // FP64 k = 32: 31 against 36 us: too few steps per tile) and for operands with
 // too few steps to hide a tile's latency (27-point 16^3 / 28^3, FP64 k = 32: 9 /
 // 15 against 12 / 13 us; FP32 36^3 / 45^3 12 / 21 against 14 / 21).

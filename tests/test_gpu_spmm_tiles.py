@@ -147,3 +147,42 @@ def test_tiles_updates_both_forms_and_trans(pls, orc, gen):
     D = np.zeros((m, k))
     np.add.at(D, ci, v[:, None] * np.repeat(Bv, np.diff(rp), axis=0))
     assert np.linalg.norm(Co.export_dense() - D) <= 1e-12 * np.linalg.norm(D)
+
+
+@pytest.mark.parametrize("warm,k", [(16, 128), (128, 16)])
+def test_first_use_of_a_form_inside_a_capture(pls, orc, warm, k):
+    """A plan warmed with one width is captured with a width of the other form."""
+    import torch
+
+    rng = np.random.default_rng(5)
+    rp, ci, v = shared_rows(rng)
+    m, n = len(rp) - 1, 1000
+    A = pls.SpMat.csr(m, n, rp, ci, v)
+    Bh = rng.uniform(-1, 1, (n, max(k, warm)))
+    B = torch.from_numpy(Bh[:, :k].copy()).cuda()
+    Bw = torch.from_numpy(Bh[:, :warm].copy()).cuda()
+    C, Cw = (torch.zeros((m, w), dtype=torch.float64, device="cuda") for w in (k, warm))
+    prev = torch.cuda.current_stream()
+    try:
+        A.spmm_async(warm, Bw.data_ptr(), warm, Cw.data_ptr(), warm)
+        torch.cuda.synchronize()
+        side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            pls.set_stream(side.cuda_stream)
+            A.spmm_async(k, B.data_ptr(), k, C.data_ptr(), k)
+    finally:
+        pls.set_stream(prev.cuda_stream)
+    mag = orc.spmm(m, k, rp, ci, np.abs(v), np.abs(Bh[:, :k]), 1.0, 0.0, None)
+    for scale in (1.0, -2.0, 0.5):  # exact scalings: eager work between the replays
+        B.copy_(torch.from_numpy(Bh[:, :k] * scale))
+        C.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = C.cpu().numpy().copy()
+        ref = orc.spmm(m, k, rp, ci, v, Bh[:, :k] * scale, 1.0, 0.0, None)
+        lim = (np.diff(rp)[:, None] + 6) * 2.0 ** -53 * abs(scale) * mag + 1e-300
+        assert (np.abs(got - ref) <= lim).all()
+    A.spmm_async(k, B.data_ptr(), k, C.data_ptr(), k)  # outside: the form is built
+    torch.cuda.synchronize()
+    assert (np.abs(C.cpu().numpy() - ref) <= lim).all()
