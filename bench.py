@@ -148,8 +148,8 @@ def cpu_baseline(n, rp, ci, v, x, y_gpu) -> dict:
 def batch_lines(nprob: int, steps: int, warmup: int, with_cpu: bool) -> dict:
     """The batched configuration: 4096 banded problems (rows log-uniform in
     [256, 65536], bandwidth 32-512, 5-40 non-zeros per row, k in {1, 4, 16}) as
-    one persistent launch replayed from a hipGraph, for FP64, FP32 and BF16
-    value storage.  GB/s = sum of every problem's algorithmic bytes / replay
+    one replay of a hipGraph, for FP64, FP32 and BF16 value storage.
+    GB/s = sum of every problem's algorithmic bytes / replay
     time; the FP32 and BF16 results are compared with the FP64 run's (the FP64
     batch itself is checked against the compensated oracle by the tests)."""
     import numpy as np

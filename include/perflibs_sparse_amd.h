@@ -276,7 +276,7 @@ perflibs_status_t perflibs_amd_sell_export(perflibs_spmat_t A, int64_t *cs,
                                            int64_t *col_indx_min,
                                            int64_t *offsets, double *vals);
 
-/* ---- batched products: one persistent launch, replayed from a hipGraph ----
+/* ---- batched products: one hipGraph replay ----
  * A batch holds nprob independent products Y_p = alpha*A_p*X_p + beta*Y_p:
  * A_p a sparse handle (CSR, or BSR / SELL-C-sigma through their CSR view),
  * NOTRANS, all of one data type; X_p (n_p x k_p) and Y_p (m_p x k_p) row-major
@@ -304,8 +304,8 @@ perflibs_status_t perflibs_amd_batch_optimize(perflibs_amd_batch_t B, int autotu
 perflibs_status_t perflibs_amd_batch_set_shape(perflibs_amd_batch_t B, perflibs_int_t tile_nnz,
                                                const perflibs_int_t *lanes,
                                                const perflibs_int_t *cpl);
-/* Enqueue the whole batch on the library stream as one kernel launch, replayed
- * from a hipGraph (captured on first use and after a change of alpha, beta or
+/* Enqueue the whole batch on the library stream as one replay of a
+ * hipGraph (captured on first use and after a change of alpha, beta or
  * shape).  Not synchronized. */
 perflibs_status_t perflibs_amd_batch_exec(perflibs_amd_batch_t B, double alpha, double beta);
 /* Run the k = 1 problems of the batch as SELL-C-sigma tiles: C = 32 or 64 rows

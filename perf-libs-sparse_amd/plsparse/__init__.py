@@ -587,7 +587,7 @@ def spmm_optimize(transA, transB, alpha_hint, A: SpMat, B: SpMat, beta_hint, Cm:
 
 class Batch:
     """A batch of CSR products Y_p = alpha*A_p*X_p + beta*Y_p run as one
-    persistent launch replayed from a hipGraph (perflibs_amd_batch_*)."""
+    replay of a hipGraph (perflibs_amd_batch_*)."""
 
     K_CLASSES = (1, 2, 4, 8, 16)
 
