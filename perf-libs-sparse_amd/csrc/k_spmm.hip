@@ -342,24 +342,28 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
 // direct kernels, which fetch a B row per non-zero.
 // Bound by the block's chain of loads and barriers and by the instructions per
 // non-zero (FP32, k = 8: vector units busy 70% of the time when every step of 8
-// masked its tail).  So a row is walked in steps of 8, 4, 2 and 1 without masks
-// (from 4 where a lane's columns take more than 16 bytes: the registers of 8
-// cost FP64 k = 16 a workgroup per CU, 98 -> 109 us), and FP32 chunks of up to
-// 16 columns keep an entry as one 8-byte LDS read, value and byte offset of its
-// B row (PACK; chunks of 32 lose a workgroup by the larger entries, 5-point 80^3
-// k = 32 47.4 -> 49.3 us).  Masked steps of 8 -> now, us: 27-point 80^3 FP32 k =
-// 8 / 16 59.1 / 66.7 -> 54.6 / 60.0, FP64 68.0 / 100.1 -> 64.9 / 97.7; 5-point
-// 1000^2 FP32 k = 8 / 32 34.2 / 66.2 -> 32.0 / 63.3; 8 x 8 block stencil FP64 k =
-// 16 50.1 -> 42.8.  A row's parts summed in contiguous pieces or four columns
-// per lane at k = 8 is slower (FP64 77 us), as is a persistent launch that
-// prefetches the next block: it loses its occupancy (FP32 k = 8 / 16 61 / 83).
+// masked its tail).  So a block's record is one load, and every load of its row
+// starts, rows, list and entries is in flight before the first LDS store; a row
+// is walked in steps of 8, 4, 2 and 1 without masks (from 4 where a lane's
+// columns take more than 16 bytes: the registers of 8 cost FP64 k = 16 a
+// workgroup per CU, 98 -> 109 us); and FP32 chunks of up to 16 columns keep an
+// entry as one 8-byte LDS read, value and byte offset of its B row (PACK; chunks
+// of 32 lose a workgroup by the larger entries, 7-point 80^3 k = 32 47 -> 49 us).
+// us, masked steps of 8 -> unmasked -> loads in flight together: 27-point 80^3
+// FP32 k = 8 / 16 59.1 / 66.7 -> 54.6 / 60.0 -> 44.6 / 51.5, FP64 68.0 / 100.1 ->
+// 64.9 / 97.7 -> 52.9 / 82.2; 5-point 1000^2 FP32 k = 8 / 32 34.2 / 66.2 -> 32.0 /
+// 63.3 -> 28.0 / 51.4; 8 x 8 block stencil FP64 k = 16 50.1 -> 42.8 -> 38.1.
+// Slower: a row's parts summed in contiguous pieces or four columns per lane at
+// k = 8 (FP64 64.9 -> 77), a persistent launch that prefetches the next block
+// (FP32 k = 8 / 16 61 / 83: it loses its occupancy), the first chunk's B loads
+// addressed from registers before the first barrier (FP64 k = 16 82 -> 99).
 // A block without a list (one row with more than UMAX distinct columns or
 // lb_nnz_per_ucol(UMAX) * UMAX non-zeros) spreads its non-zeros over the
 // workgroup's lane groups, reads B directly and sums the groups through LDS.
 template <int KC, int UMAX, int CPL, class V, class X, bool BETA>
 __global__ __launch_bounds__(kBlock) void k_spmm_lds(
-    const int32_t *__restrict__ row0s, const int32_t *__restrict__ uoff,
-    const int32_t *__restrict__ ucol, const uint8_t *__restrict__ lidx,
+    const pls::SpmmBlock *__restrict__ blocks, const int32_t *__restrict__ ucol,
+    const uint8_t *__restrict__ lidx,
     const int32_t *__restrict__ brow, const int32_t *__restrict__ prp,
     const V *__restrict__ lval, int32_t k, const int32_t *__restrict__ rp,
     const int32_t *__restrict__ ci, const V *__restrict__ val, const X *__restrict__ B,
@@ -377,13 +381,11 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
   __shared__ int32_t s_row[pls::kLbRows];  // clustered blocks: the rows' indices
   const uint32_t blk = xcd_swizzle(blockIdx.x, gridDim.x);
   const int tid = threadIdx.x, lane = tid % KC, grp = tid / KC;
-  // r0: first entry of the row order; the block's non-zeros are [e0, e0 + nnz)
-  // of the block-order arrays (the CSR arrays for consecutive rows)
-  const int32_t r0 = row0s[blk], nrows = row0s[blk + 1] - r0;
-  const int32_t u0 = uoff[blk], nu = uoff[blk + 1] - u0;
+  const pls::SpmmBlock bk = blocks[blk];
+  const int32_t r0 = bk.r0, nrows = bk.nrows, nu = bk.nu, e0 = bk.e0, nnz = bk.nnz;
+  // block-order arrays (the CSR arrays for consecutive rows)
   const int32_t *brp = brow ? prp : rp;
   const V *bval = brow ? lval : val;
-  const int32_t e0 = brp[r0], nnz = brp[r0 + nrows] - e0;
 
   if (nu == 0 && nnz > 0) {  // one long row without a list: B read directly
     const int32_t row = brow ? brow[r0] : r0, f0 = rp[row];  // its CSR non-zeros
@@ -408,33 +410,44 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
   }
 
   {
-    // values and list positions in aligned pairs from the even index at or
-    // below e0 (value and position arrays end with one padding entry)
-    const int32_t a0 = e0 & ~1, sh = e0 - a0;
+    // every load of the block's row starts, rows, list and entries in flight
+    // before the first LDS store; values and list positions in aligned pairs
+    // from the even index at or below e0 (both arrays end with one padding entry)
+    constexpr int NP = NNZ / 2 / kBlock + 1;
+    static_assert(pls::kLbRows < kBlock && UMAX <= kBlock);
     typedef uint8_t L2 __attribute__((ext_vector_type(2)));
-    for (int32_t t = tid; 2 * t < nnz + sh; t += kBlock) {
-      A v[2];
-      const int32_t j = a0 + 2 * t;
-      ld_val_pair(bval, j, v);
-      const L2 l = *reinterpret_cast<const L2 *>(lidx + j);
-      const int32_t q = 2 * t - sh;
-      auto put = [&](int32_t at, A a, uint8_t pos) {
-        if constexpr (PACK) {
-          s_e[at] = make_uint2(__float_as_uint(alpha * a), pos * uint32_t(KC * sizeof(A)));
-        } else {
-          s_a[at] = alpha * a;
-          s_l[at] = pos;
-        }
-      };
-      if (q >= 0) put(q, v[0], l.x);
-      if (q + 1 < nnz) put(q + 1, v[1], l.y);
+    const int32_t start = brp[r0 + min(tid, nrows)];
+    const int32_t row = brow ? brow[r0 + min(tid, nrows - 1)] : 0;
+    const int32_t uc = nu > 0 ? ucol[bk.u0 + min(tid, nu - 1)] : 0;
+    const int32_t a0 = e0 & ~1, sh = e0 - a0, last = (e0 + nnz - 1) & ~1;
+    A v[NP][2];
+    L2 l[NP];
+    if (nnz > 0)
+#pragma unroll
+      for (int u = 0; u < NP; ++u) {
+        const int32_t j = min(a0 + 2 * (tid + u * kBlock), last);
+        ld_val_pair(bval, j, v[u]);
+        l[u] = *reinterpret_cast<const L2 *>(lidx + j);
+      }
+    if (tid <= nrows) s_rp[tid] = start - e0;
+    if (brow && tid < nrows) s_row[tid] = row;
+    if (tid < nu) s_uc[tid] = uc;
+    auto put = [&](int32_t at, A a, uint8_t pos) {
+      if (at < 0 || at >= nnz) return;
+      if constexpr (PACK) {
+        s_e[at] = make_uint2(__float_as_uint(alpha * a), pos * uint32_t(KC * sizeof(A)));
+      } else {
+        s_a[at] = alpha * a;
+        s_l[at] = pos;
+      }
+    };
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int32_t q = 2 * (tid + u * kBlock) - sh;
+      put(q, v[u][0], l[u].x);
+      put(q + 1, v[u][1], l[u].y);
     }
   }
-  for (int32_t q = tid; q <= nrows; q += kBlock) {
-    s_rp[q] = brp[r0 + q] - e0;
-    if (brow && q < nrows) s_row[q] = brow[r0 + q];
-  }
-  for (int32_t q = tid; q < nu; q += kBlock) s_uc[q] = ucol[u0 + q];
   __syncthreads();
   // compute mapping: G = KC / CPL lanes per row group, CPL adjacent columns
   // per lane (read from LDS as one vector); S groups of one wave share a row
@@ -1146,8 +1159,7 @@ void launch_lds(const pls::DevCsr &A, int32_t k, double alpha, const void *B, in
                 double beta, void *C, int64_t ldc, hipStream_t s) {
   auto go = [&](auto kc, auto um) {
     constexpr int KC = decltype(kc)::value, UMAX = decltype(um)::value;
-    const auto *row0 = A.lb_row0.as<int32_t>();
-    const auto *uoff = A.lb_uoff.as<int32_t>();
+    const auto *blocks = A.lb_block.as<pls::SpmmBlock>();
     const auto *ucol = A.lb_ucol.as<int32_t>();
     const auto *lidx = A.lb_lidx.as<uint8_t>();
     // clustered blocks (nullptr for consecutive rows): row order, block-order
@@ -1157,11 +1169,11 @@ void launch_lds(const pls::DevCsr &A, int32_t k, double alpha, const void *B, in
     const auto *lval = A.lb_val.as<V>();
     if (beta != 0.0)
       k_spmm_lds<KC, UMAX, (KC >= 16 ? 4 : 2), V, X, true><<<A.lb_nblocks, kBlock, 0, s>>>(
-          row0, uoff, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
+          blocks, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
           A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(beta));
     else
       k_spmm_lds<KC, UMAX, (KC >= 16 ? 4 : 2), V, X, false><<<A.lb_nblocks, kBlock, 0, s>>>(
-          row0, uoff, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
+          blocks, ucol, lidx, brow, prp, lval, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(),
           A.vals.as<V>(), (const X *)B, ldb, (X *)C, ldc, acc_t<X>(alpha), acc_t<X>(0));
   };
   // Column chunks: 8 for k <= 8 and for FP64 lists of 256, then 16 (FP64) or

@@ -106,6 +106,12 @@ struct LbHost;  // host form of the SpMM row blocks (spmm_blocks.cpp)
 struct SpmmTile {
   int32_t row0, step0, val0, half;
 };
+// A block of the LDS form: entries [r0, r0 + nrows) of the row order, its list
+// ucol[u0 .. u0 + nu) and its non-zeros [e0, e0 + nnz) in block order; nu = 0
+// with nnz > 0 is one long row without a list.
+struct SpmmBlock {
+  int32_t r0, nrows, u0, nu, e0, nnz;
+};
 // Values past the last tile that k_spmm_tile may read ahead.
 constexpr int32_t kTilePad = 512;
 // Non-zeros of a row above which k_spmm_gather gives it a workgroup of its own
@@ -136,8 +142,7 @@ struct DevCsr {
   int32_t lb_umax = 0;   // list length limit the blocks were cut with
   int64_t lb_ucols = 0;  // total list length (sum of distinct columns per block)
   bool lb_clustered = false;  // blocks of clustered rows (lb_brow holds them)
-  DevBuf lb_row0;        // int32 [nb+1] block b: entries [row0[b], row0[b+1]) of the row order
-  DevBuf lb_uoff;        // int32 [nb+1] offsets into lb_ucol
+  DevBuf lb_block;       // SpmmBlock [lb_nblocks]
   DevBuf lb_ucol;        // int32 [lb_ucols]
   DevBuf lb_lidx;        // uint8 [nnz] (block order when clustered)
   DevBuf lb_brow;        // int32 [m] row order of clustered blocks (empty: row i is entry i)
@@ -179,7 +184,7 @@ constexpr int32_t kLbRows = 128;
 // often but need no barriers, and multiply on the matrix cores (27-point
 // stencil 80^3, FP64 k = 32 / 128: 168 / 555 -> 118 / 409 us, FP32 k = 64 / 128
 // 155 / 276 -> 111 / 214).  LDS stays faster for k <= 16 (half of a 32-column
-// product idle: FP64 k = 16 98 against 106 us), for short rows (5-point 500^2,
+// product idle: FP64 k = 16 82 against 106 us), for short rows (5-point 500^2,
 // FP64 k = 32: 31 against 36 us: too few steps per tile) and for operands with
 // too few steps to hide a tile's latency (27-point 16^3 / 28^3, FP64 k = 32: 9 /
 // 15 against 12 / 13 us; FP32 36^3 / 45^3 12 / 21 against 14 / 21).

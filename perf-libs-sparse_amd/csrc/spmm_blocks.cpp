@@ -361,10 +361,9 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
   d.lb_prp.reset();
   d.lb_epos.reset();
   d.lb_val.reset();
-  hipError_t e = d.lb_row0.upload(h.row0.data(), sizeof(int32_t) * h.row0.size());
-  if (e == hipSuccess) e = d.lb_uoff.upload(h.uoff.data(), sizeof(int32_t) * h.uoff.size());
-  if (e == hipSuccess)
-    e = d.lb_ucol.upload(h.ucol.data(), sizeof(int32_t) * std::max<size_t>(h.ucol.size(), 1));
+  hipError_t e =
+      d.lb_ucol.upload(h.ucol.data(), sizeof(int32_t) * std::max<size_t>(h.ucol.size(), 1));
+  std::vector<int32_t> prp;  // clustered: first non-zero of each entry of the row order
   // list positions and block-order values end with one padding entry (the
   // kernel stages them in aligned pairs); the CSR plan's values carry theirs
   if (h.brow.empty()) {
@@ -374,7 +373,8 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
   } else {
     const int32_t m = o.m, base = o.prp[0];
     const size_t nnz = h.lidx.size();
-    std::vector<int32_t> prp(size_t(m) + 1, 0), epos(nnz + 1, 0);
+    prp.assign(size_t(m) + 1, 0);
+    std::vector<int32_t> epos(nnz + 1, 0);
     std::vector<uint8_t> lidx(nnz + 1, 0);
     for (int32_t i = 0; i < m; ++i) {
       const int32_t r = h.brow[size_t(i)];
@@ -402,6 +402,14 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
       e = plk::gather_vals(d.vs, d.lb_val.get(), d.vals.get(), d.lb_epos.as<int32_t>(),
                            int64_t(nnz + 1), stream());
   }
+  const auto first = [&](int32_t r) { return h.brow.empty() ? o.prp[r] - o.prp[0] : prp[size_t(r)]; };
+  std::vector<SpmmBlock> blocks(h.row0.size() - 1);
+  for (size_t b = 0; b < blocks.size(); ++b) {
+    const int32_t r0 = h.row0[b], r1 = h.row0[b + 1], u0 = h.uoff[b];
+    blocks[b] = {r0, r1 - r0, u0, h.uoff[b + 1] - u0, first(r0), first(r1) - first(r0)};
+  }
+  if (e == hipSuccess)
+    e = d.lb_block.upload(blocks.data(), sizeof(SpmmBlock) * std::max<size_t>(blocks.size(), 1));
   d.lb_lds = e == hipSuccess;
   return e;
 }
