@@ -182,15 +182,19 @@ constexpr int32_t kLbRows = 128;
 // Whether a product with k columns runs on the row tiles (k_spmm_tile) or
 // stages the blocks' B rows in LDS (k_spmm_lds).  Tiles read a B row about as
 // often but need no barriers, and multiply on the matrix cores (27-point
-// stencil 80^3, FP64 k = 32 / 128: 168 / 555 -> 118 / 409 us, FP32 k = 64 / 128
-// 155 / 276 -> 111 / 214).  LDS stays faster for k <= 16 (half of a 32-column
-// product idle: FP64 k = 16 82 against 106 us), for short rows (5-point 500^2,
-// FP64 k = 32: 31 against 36 us: too few steps per tile) and for operands with
-// too few steps to hide a tile's latency (27-point 16^3 / 28^3, FP64 k = 32: 9 /
-// 15 against 12 / 13 us; FP32 36^3 / 45^3 12 / 21 against 14 / 21).
+// stencil 80^3, LDS against tiles, FP64 k = 32 / 64 / 128: 157 / 282 / 497 against
+// 122 / 217 / 407 us, FP32 k = 64 / 128 138 / 239 against 118 / 215).  LDS is
+// faster for k <= 16 (half of a 32-column product idle: FP64 k = 16 82 against 106
+// us), for FP32 of up to 32 columns, one LDS chunk, unless rows are long (27-point
+// 80^3 / 64^3, 27 non-zeros per row, k = 32: 69 / 40 against 79 / 48; 4 x 4 and
+// 8 x 8 block stencils, 108 and 216 per row: 37 and 38 against 32 and 30), for
+// short rows (5-point 500^2, FP64 k = 32: 27 against 36 us: too few steps per
+// tile) and for operands with too few steps to hide a tile's latency (27-point
+// 28^3, 114k listed columns, FP64 k = 32 / 48: 11.6 / 16.2 against 13.2 / 18.2 us;
+// 36^3, 242k: 19.4 / 26.4 against 18.9 / 26.9).
 inline bool spmm_on_tiles(const DevCsr &d, bool dbl, int64_t k) {
-  return d.lb_state == 1 && k > 16 && d.nnz >= 10 * int64_t(d.m) &&
-         (k > 64 || d.lb_ucols >= (dbl || k > 32 ? 100000 : 320000));
+  return d.lb_state == 1 && k > 16 && d.nnz >= (dbl || k > 32 ? 10 : 64) * int64_t(d.m) &&
+         (k > 64 || d.lb_ucols >= (dbl || k > 32 ? 160000 : 320000));
 }
 
 // Device SELL-C-sigma (layout of src/sell_c_sigma.hpp:43-104, NOTRANS).

@@ -186,3 +186,15 @@ def test_first_use_of_a_form_inside_a_capture(pls, orc, warm, k):
     A.spmm_async(k, B.data_ptr(), k, C.data_ptr(), k)  # outside: the form is built
     torch.cuda.synchronize()
     assert (np.abs(C.cpu().numpy() - ref) <= lim).all()
+
+
+@pytest.mark.parametrize("k", [65, 96, 97, 161])
+def test_narrow_window_for_the_rest(pls, orc, k):
+    """Enough listed columns (320000) for a second launch: rests of 1, 32 and 33."""
+    rng = np.random.default_rng(8)
+    m, per = 100000, 20
+    lo = np.minimum(np.maximum(np.arange(m) - 50, 0), m - 100)
+    ci = (lo[:, None] + 5 * np.arange(per)[None, :] + rng.integers(0, 5, (m, per))).astype(np.int32)
+    rp = (per * np.arange(m + 1)).astype(np.int32)
+    bad = [(1000, k - 1, np.inf), (2000, 64, np.nan), (3000, 63, np.inf)]
+    check(pls, orc, rp, ci.ravel(), rng.standard_normal(m * per), m, k, "f64", 0.5, bad=bad)
