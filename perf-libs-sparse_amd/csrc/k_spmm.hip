@@ -177,7 +177,7 @@ __device__ __forceinline__ void store_cols(X *crow, int64_t c0, int64_t own, int
 // Bound: 27-point stencil 96^3, FP64 k = 32, 203 us (floor 156 at the copy rate,
 // matrix cores 106), k = 128 on 80^3 408 us (floor 257): matrix cores about half
 // busy and 2.5 GB moved for 1.2 GB, B rows fetched again across grid planes.
-// k_spmm_lds takes 275 and 553 us there.
+// k_spmm_lds took 275 and 553 us there, with its present staging 497 at k = 128.
 // A wave whose results hold a NaN computes them again entry by entry: a column
 // some row of the tile does not have is multiplied by zero for that row, which
 // changes nothing unless the B value is infinite or NaN.
