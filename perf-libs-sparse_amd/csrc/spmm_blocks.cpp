@@ -353,6 +353,19 @@ bool cut_clustered(const Operand &o, int32_t umax, const std::vector<int32_t> &c
   return int32_t(h.brow.size()) == m;
 }
 
+// A form's values gathered from the plan's, on a stream of its own and waited
+// for: whichever stream the next product runs on, it finds them written.  (The
+// plan's values themselves are complete: their uploads and updates wait.)
+hipError_t gather_and_wait(VStore vs, void *dst, const DevCsr &d, const DevBuf &epos, int64_t n) {
+  hipStream_t s = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  if (e != hipSuccess) return e;
+  e = plk::gather_vals(vs, dst, d.vals.get(), epos.as<int32_t>(), n, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipStreamDestroy(s);
+  return e;
+}
+
 // Clustered blocks also keep their non-zeros in block order: first non-zero
 // of each entry of the row order (prp), list positions, the CSR position of
 // each (epos) and the values gathered through it on the device.
@@ -398,9 +411,7 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
     epos[nnz] = int32_t(nnz);
     if (e == hipSuccess) e = d.lb_epos.upload(epos.data(), sizeof(int32_t) * (nnz + 1));
     if (e == hipSuccess) e = d.lb_val.alloc(es * (nnz + 1));
-    if (e == hipSuccess)
-      e = plk::gather_vals(d.vs, d.lb_val.get(), d.vals.get(), d.lb_epos.as<int32_t>(),
-                           int64_t(nnz + 1), stream());
+    if (e == hipSuccess) e = gather_and_wait(d.vs, d.lb_val.get(), d, d.lb_epos, int64_t(nnz + 1));
   }
   const auto first = [&](int32_t r) { return h.brow.empty() ? o.prp[r] - o.prp[0] : prp[size_t(r)]; };
   std::vector<SpmmBlock> blocks(h.row0.size() - 1);
@@ -538,9 +549,7 @@ hipError_t upload_tiles(const Operand &o, const LbHost &h, DevCsr &d) {
   if (e == hipSuccess) e = d.t_val.alloc(es * (nv + size_t(kTilePad)));
   d.t_nnz = int64_t(nv);
   d.t_ndirect = int32_t(nd);
-  if (e == hipSuccess)
-    e = plk::gather_vals(d.vs, d.t_val.get(), d.vals.get(), d.t_epos.as<int32_t>(),
-                         d.t_nnz + kTilePad, stream());
+  if (e == hipSuccess) e = gather_and_wait(d.vs, d.t_val.get(), d, d.t_epos, d.t_nnz + kTilePad);
   d.ntiles = e == hipSuccess ? int32_t(nt) : -1;
   return e;
 }
