@@ -354,8 +354,8 @@ perflibs_status_t spmm(int transA, int transB, T alpha, perflibs_spmat_top_t *A,
   if (!exec) return PERFLIBS_STATUS_SUCCESS;
 
   // op(B) row-major view: NOTRANS row-major B, or TRANS column-major B
-  e = plk::csr_spmm(*A->plan.csr, dbl, n, double(alpha), bd.dev.get(), bd.lda, 1, double(beta),
-                    cd.dev.get(), cd.lda, 1, s);
+  e = plk::csr_spmm(*A->plan.csr, dbl, n, double(alpha), bd.dev.get(), bd.lda, double(beta),
+                    cd.dev.get(), cd.lda, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM");
   cd.host_valid = false;
@@ -381,8 +381,8 @@ perflibs_status_t spmm_async(T alpha, perflibs_spmat_top_t *A, perflibs_int_t k,
   }
   st = csr_plan_for(A, PERFLIBS_SPARSE_OPERATION_NOTRANS, k);
   if (st != PERFLIBS_STATUS_SUCCESS) return st;
-  e = plk::csr_spmm(*A->plan.csr, dt == DType::F64, k, double(alpha), B, ldb, 1, double(beta), C,
-                    ldc, 1, pls::stream());
+  e = plk::csr_spmm(*A->plan.csr, dt == DType::F64, k, double(alpha), B, ldb, double(beta), C,
+                    ldc, pls::stream());
   if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM");
   return PERFLIBS_STATUS_SUCCESS;
 }

@@ -4,9 +4,8 @@
 // (spmm_rowwise_csr_blocked_m_kernel, src/compressed_sparse_rows.cpp:1699-1745,
 // and the C zeroing of src/matmul.cpp:596-605): beta == 0 never reads C.
 //
-// Row-major B and C: k_spmm_tile or k_spmm_lds where a block of rows shares its
-// B rows, else k_spmm_gather.  Strided (column-major / transposed) operands use the generic
-// kernel, one thread per output element.
+// B and C are row-major (the driver lays others out again first): k_spmm_tile or
+// k_spmm_lds where a block of rows shares its B rows, else k_spmm_gather.
 #include <algorithm>
 #include <type_traits>
 
@@ -576,23 +575,6 @@ __global__ __launch_bounds__(kBlock) void k_spmm_lds(
     }
     __syncthreads();
   }
-}
-
-template <class V, class X, bool BETA>
-__global__ __launch_bounds__(kBlock) void k_spmm_strided(
-    int32_t m, int32_t k, const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
-    const V *__restrict__ val, const X *__restrict__ B, int64_t b_sr, int64_t b_sc,
-    X *__restrict__ Cm, int64_t c_sr, int64_t c_sc, acc_t<X> alpha, acc_t<X> beta) {
-  using A = acc_t<X>;
-  const int64_t t = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  if (t >= int64_t(m) * k) return;
-  const int64_t i = t / k, j = t % k;
-  A s = 0;
-  for (int32_t p = rp[i]; p < rp[i + 1]; ++p) s += A(ldv(val, p)) * A(B[int64_t(ci[p]) * b_sr + j * b_sc]);
-  X *c = Cm + i * c_sr + j * c_sc;
-  A r = alpha * s;
-  if (BETA) r += beta * A(*c);
-  *c = X(r);
 }
 
 // Few right-hand sides (n < 5, the range where the reference repeats SpMV per
@@ -1206,30 +1188,18 @@ void launch_lds(const pls::DevCsr &A, int32_t k, double alpha, const void *B, in
 }  // namespace
 
 hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, const void *B,
-                    int64_t b_sr, int64_t b_sc, double beta, void *C, int64_t c_sr,
-                    int64_t c_sc, hipStream_t s) {
+                    int64_t ldb, double beta, void *C, int64_t ldc, hipStream_t s) {
   if (A.m == 0 || k == 0) return hipSuccess;
   auto run = [&](auto vtag, auto xtag) -> hipError_t {
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
-    const bool rm = b_sc == 1 && c_sc == 1;
-    if (rm && pls::spmm_on_tiles(A, dbl, k) && A.ntiles >= 0) {
-      dispatch_tile<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
-      dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s, true);
-    } else if (rm && k >= 8 && A.lb_lds && A.lb_nblocks > 0) {
-      launch_lds<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s);
-    } else if (rm) {
-      dispatch_gather<V, X>(A, k, alpha, B, b_sr, beta, C, c_sr, s, false);
+    if (pls::spmm_on_tiles(A, dbl, k) && A.ntiles >= 0) {
+      dispatch_tile<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+      dispatch_gather<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, true);
+    } else if (k >= 8 && A.lb_lds && A.lb_nblocks > 0) {
+      launch_lds<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
     } else {
-      const unsigned grid = grid_for(int64_t(A.m) * k);
-      if (beta != 0.0)
-        k_spmm_strided<V, X, true><<<grid, kBlock, 0, s>>>(
-            A.m, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, b_sr,
-            b_sc, (X *)C, c_sr, c_sc, acc_t<X>(alpha), acc_t<X>(beta));
-      else
-        k_spmm_strided<V, X, false><<<grid, kBlock, 0, s>>>(
-            A.m, k, A.rp.as<int32_t>(), A.ci.as<int32_t>(), A.vals.as<V>(), (const X *)B, b_sr,
-            b_sc, (X *)C, c_sr, c_sc, acc_t<X>(alpha), acc_t<X>(0));
+      dispatch_gather<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, false);
     }
     return hipGetLastError();
   };

@@ -99,7 +99,6 @@ struct Dense {
   bool matrix_is_zero = false;
 };
 
-// Device CSR (0-based) with the row-block table of the adaptive kernel.
 struct LbHost;  // host form of the SpMM row blocks (spmm_blocks.cpp)
 // A tile of at most 32 rows in two halves: its first row, step and value (the
 // next tile's end them) and the rows of the first half.
@@ -118,6 +117,7 @@ constexpr int32_t kTilePad = 512;
 // (power-law 1M rows, FP64 k = 8 / 64: 411 / 1702 us with 128, 387 / 1608 with
 // 256, 380 / 1577 with 512).
 constexpr int32_t kSpmmLongRow = 512;
+// Device CSR (0-based) with the row-block table of the adaptive kernel.
 struct DevCsr {
   int32_t m = 0, n = 0;
   int64_t nnz = 0;
@@ -510,15 +510,13 @@ hipError_t scale_vec(bool dbl, int64_t n, double beta, void *y, hipStream_t s);
 // y = alpha*x + beta*y.
 hipError_t axpby_vec(bool dbl, int64_t n, double alpha, const void *x, double beta,
                      void *y, hipStream_t s);
-// C(i,j) = alpha * sum A(i,p) B(p,j) + beta*C(i,j) (beta==0: C ignored) with
-// B(r,c) at B[r*bsr + c*bsc] and C(r,c) at C[r*csr + c*csc].
-hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha,
-                    const void *B, int64_t b_sr, int64_t b_sc, double beta, void *C,
-                    int64_t c_sr, int64_t c_sc, hipStream_t s);
+// C = alpha*A*B + beta*C (beta == 0: C is not read), B and C row-major with
+// leading dimensions ldb and ldc.
+hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, const void *B,
+                    int64_t ldb, double beta, void *C, int64_t ldc, hipStream_t s);
 // Scale a strided m x n dense matrix by beta (beta == 0: set to zero).
 hipError_t scale_dense(bool dbl, int64_t m, int64_t n, double beta, void *C,
                        int64_t sr, int64_t sc, hipStream_t s);
-// dst[i*ds] = src[i*ss], i < n.
 // C = alpha*A*B + beta*C on BSR blocks (b = 4 or 8), B and C row-major with
 // leading dimensions ldb and ldc; stored zeros add nothing.
 hipError_t bsr_spmm(const pls::DevBsr &A, bool dbl, int32_t k, double alpha, const void *B,
@@ -529,6 +527,7 @@ hipError_t bsr_spmm(const pls::DevBsr &A, bool dbl, int32_t k, double alpha, con
 int few_rhs_pitch(int32_t n);
 hipError_t csr_spmm_few(const pls::DevCsr &A, bool dbl, int32_t n, double alpha, const void *B,
                         double beta, void *C, int64_t c_sr, int64_t c_sc, hipStream_t s);
+// dst[i*ds] = src[i*ss], i < n.
 hipError_t strided_copy(bool dbl, int64_t n, const void *src, int64_t ss, void *dst, int64_t ds,
                         hipStream_t s);
 // FP32 -> BF16 (round to nearest even), n values, device to device.
