@@ -149,31 +149,36 @@ perflibs_status_t to_csr_keeping_blocks(perflibs_spmat_top_t *A, bool keep) {
 
 // CSR plan of op(A) for SpMM with k columns of B; for k >= 8 also the
 // column-compressed row blocks (cut once per plan) in the form that product
-// runs on.
-perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k) {
+// runs on.  The form is chosen under the plan's lock: one that another thread
+// adds meanwhile does not change this product's kernel.
+perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k, pls::SpmmForm &form) {
+  form = pls::SpmmForm::Gather;
   pls::Operand o;
   if (!(A->plan.csr && A->plan.op == op)) {
     if (!pls::make_operand(A, op, o)) return pls::exec_fail(A, "matrix format has no GPU SpMM path");
     const perflibs_status_t st = pls::build_plan(A, o, op, PERFLIBS_AMD_CSR_VECTOR);
     if (st != PERFLIBS_STATUS_SUCCESS) return st;
   }
+  if (k < 8) return PERFLIBS_STATUS_SUCCESS;
   pls::DevCsr &d = *A->plan.csr;
-  if (k < 8 || d.lb_state < 0) return PERFLIBS_STATUS_SUCCESS;
   auto tiles = [&] { return pls::spmm_on_tiles(d, A->dt == DType::F64, k); };
-  // one thread builds a form; a product on the other form does not touch it
   const std::lock_guard<std::mutex> lock(d.lb_mutex);
-  if (d.lb_state == 0 || (tiles() ? d.ntiles < 0 : !d.lb_lds)) {
-    // no allocation or copy inside a capture: csr_spmm takes the form that is there
+  if (d.lb_state < 0) return PERFLIBS_STATUS_SUCCESS;
+  if (d.lb_state == 0 || !d.has_form(tiles())) {
+    // no allocation or copy inside a capture: the form that is there, if it serves
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (d.lb_state == 1 && (d.ntiles >= 0 || d.lb_lds) &&
-        hipStreamIsCapturing(pls::stream(), &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
-      return PERFLIBS_STATUS_SUCCESS;
-    if (!o.prp && !pls::make_operand(A, op, o))
-      return pls::exec_fail(A, "matrix format has no GPU SpMM path");
-    if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);
-    const hipError_t e = pls::upload_spmm_form(o, d, tiles());
-    if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM block upload");
+    const bool other = d.lb_state == 1 && d.has_form(!tiles());
+    if (!(other && hipStreamIsCapturing(pls::stream(), &cs) == hipSuccess &&
+          cs != hipStreamCaptureStatusNone)) {
+      if (!o.prp && !pls::make_operand(A, op, o))
+        return pls::exec_fail(A, "matrix format has no GPU SpMM path");
+      if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);
+      const hipError_t e = pls::upload_spmm_form(o, d, tiles());
+      if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM block upload");
+    }
   }
+  if (tiles() && d.has_form(true)) form = pls::SpmmForm::Tiles;
+  else if (d.has_form(false)) form = pls::SpmmForm::Lds;
   return PERFLIBS_STATUS_SUCCESS;
 }
 
@@ -349,12 +354,13 @@ perflibs_status_t spmm(int transA, int transB, T alpha, perflibs_spmat_top_t *A,
     cd.matrix_is_zero = false;
     return PERFLIBS_STATUS_SUCCESS;
   }
-  st = csr_plan_for(A, transA, n);
+  pls::SpmmForm form;
+  st = csr_plan_for(A, transA, n, form);
   if (st != PERFLIBS_STATUS_SUCCESS) return st;
   if (!exec) return PERFLIBS_STATUS_SUCCESS;
 
   // op(B) row-major view: NOTRANS row-major B, or TRANS column-major B
-  e = plk::csr_spmm(*A->plan.csr, dbl, n, double(alpha), bd.dev.get(), bd.lda, double(beta),
+  e = plk::csr_spmm(*A->plan.csr, dbl, form, n, double(alpha), bd.dev.get(), bd.lda, double(beta),
                     cd.dev.get(), cd.lda, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM");
@@ -379,10 +385,11 @@ perflibs_status_t spmm_async(T alpha, perflibs_spmat_top_t *A, perflibs_int_t k,
     if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM");
     return PERFLIBS_STATUS_SUCCESS;
   }
-  st = csr_plan_for(A, PERFLIBS_SPARSE_OPERATION_NOTRANS, k);
+  pls::SpmmForm form;
+  st = csr_plan_for(A, PERFLIBS_SPARSE_OPERATION_NOTRANS, k, form);
   if (st != PERFLIBS_STATUS_SUCCESS) return st;
-  e = plk::csr_spmm(*A->plan.csr, dt == DType::F64, k, double(alpha), B, ldb, double(beta), C,
-                    ldc, pls::stream());
+  e = plk::csr_spmm(*A->plan.csr, dt == DType::F64, form, k, double(alpha), B, ldb, double(beta),
+                    C, ldc, pls::stream());
   if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM");
   return PERFLIBS_STATUS_SUCCESS;
 }

@@ -1187,16 +1187,16 @@ void launch_lds(const pls::DevCsr &A, int32_t k, double alpha, const void *B, in
 
 }  // namespace
 
-hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, const void *B,
-                    int64_t ldb, double beta, void *C, int64_t ldc, hipStream_t s) {
+hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, pls::SpmmForm form, int32_t k, double alpha,
+                    const void *B, int64_t ldb, double beta, void *C, int64_t ldc, hipStream_t s) {
   if (A.m == 0 || k == 0) return hipSuccess;
   auto run = [&](auto vtag, auto xtag) -> hipError_t {
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
-    if (pls::spmm_on_tiles(A, dbl, k) && A.ntiles >= 0) {
+    if (form == pls::SpmmForm::Tiles) {
       dispatch_tile<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       dispatch_gather<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, true);
-    } else if (k >= 8 && A.lb_lds && A.lb_nblocks > 0) {
+    } else if (form == pls::SpmmForm::Lds) {
       launch_lds<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
     } else {
       dispatch_gather<V, X>(A, k, alpha, B, ldb, beta, C, ldc, s, false);

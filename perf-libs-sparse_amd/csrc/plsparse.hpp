@@ -117,6 +117,9 @@ constexpr int32_t kTilePad = 512;
 // (power-law 1M rows, FP64 k = 8 / 64: 411 / 1702 us with 128, 387 / 1608 with
 // 256, 380 / 1577 with 512).
 constexpr int32_t kSpmmLongRow = 512;
+// The kernel a CSR x dense product runs on: B rows gathered per non-zero, or the
+// row blocks staged in LDS, or their row tiles.
+enum class SpmmForm { Gather, Lds, Tiles };
 // Device CSR (0-based) with the row-block table of the adaptive kernel.
 struct DevCsr {
   int32_t m = 0, n = 0;
@@ -151,9 +154,10 @@ struct DevCsr {
   DevBuf lb_val;         // [nnz] vals in block order, storage vs (clustered; refreshed by updates)
   std::shared_ptr<LbHost> lb_host;  // the cut, from which either form below is built on first use
   bool lb_lds = false;              // the arrays above are on the device (k_spmm_lds)
-  std::mutex lb_mutex;              // held while a form is built
+  std::mutex lb_mutex;              // held while a form is chosen or built
   // Row tiles of the blocks (k_spmm_tile), on the device when ntiles >= 0
   int32_t ntiles = -1, t_ndirect = 0;
+  bool has_form(bool tiles) const { return lb_state == 1 && (tiles ? ntiles >= 0 : lb_lds); }
   int64_t t_nnz = 0;  // non-zeros of the tiles
   DevBuf t_tiles;     // SpmmTile [ntiles + 1]
   DevBuf t_row;       // int32 rows, tile by tile
@@ -511,9 +515,9 @@ hipError_t scale_vec(bool dbl, int64_t n, double beta, void *y, hipStream_t s);
 hipError_t axpby_vec(bool dbl, int64_t n, double alpha, const void *x, double beta,
                      void *y, hipStream_t s);
 // C = alpha*A*B + beta*C (beta == 0: C is not read), B and C row-major with
-// leading dimensions ldb and ldc.
-hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, int32_t k, double alpha, const void *B,
-                    int64_t ldb, double beta, void *C, int64_t ldc, hipStream_t s);
+// leading dimensions ldb and ldc, on a form that is on the device.
+hipError_t csr_spmm(const pls::DevCsr &A, bool dbl, pls::SpmmForm form, int32_t k, double alpha,
+                    const void *B, int64_t ldb, double beta, void *C, int64_t ldc, hipStream_t s);
 // Scale a strided m x n dense matrix by beta (beta == 0: set to zero).
 hipError_t scale_dense(bool dbl, int64_t m, int64_t n, double beta, void *C,
                        int64_t sr, int64_t sc, hipStream_t s);

@@ -79,3 +79,22 @@ for i in at:
 later = product({k}, S2)
 assert not any("k_gather_vals" in f for f in kernels(later)) and form(later) == form(calls)
 """)
+
+
+def test_threads_share_a_plan(run):
+    """Products of both widths from several threads on one warmed handle: each
+    form is built once, and every product runs on the form of its width."""
+    run("""
+import threading
+product(8)
+stub.stub_clear()
+P.set_stream(S1)
+def work(k):
+    for _ in range(50):
+        A.spmm_async(k, buf.ctypes.data, k, buf.ctypes.data, k)
+ts = [threading.Thread(target=work, args=(k,)) for k in (128, 16, 128, 16)]
+[t.start() for t in ts], [t.join() for t in ts]
+ran = kernels([tuple(x.split()) for x in stub.stub_log().decode().splitlines()])
+assert sum("k_spmm_tile" in f for f in ran) == 100 and sum("k_spmm_lds" in f for f in ran) == 100
+assert sum("k_gather_vals" in f for f in ran) == 1  # the tiles' values
+""")
