@@ -147,6 +147,22 @@ perflibs_status_t to_csr_keeping_blocks(perflibs_spmat_top_t *A, bool keep) {
   return PERFLIBS_STATUS_SUCCESS;
 }
 
+// Allows this thread what a capture forbids: allocations, work on other streams.
+class RelaxedCapture {
+ public:
+  explicit RelaxedCapture(bool on) : on_(on) { swap(); }
+  ~RelaxedCapture() { swap(); }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+  RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+
+ private:
+  void swap() {
+    if (on_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+  const bool on_;
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // CSR plan of op(A) for SpMM with k columns of B; for k >= 8 also the
 // column-compressed row blocks (cut once per plan) in the form that product
 // runs on.  The form is chosen under the plan's lock: one that another thread
@@ -165,17 +181,16 @@ perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k, pls::
   const std::lock_guard<std::mutex> lock(d.lb_mutex);
   if (d.lb_state < 0) return PERFLIBS_STATUS_SUCCESS;
   if (d.lb_state == 0 || !d.has_form(tiles())) {
-    // no allocation or copy inside a capture: the form that is there, if it serves
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool other = d.lb_state == 1 && d.has_form(!tiles());
-    if (!(other && hipStreamIsCapturing(pls::stream(), &cs) == hipSuccess &&
-          cs != hipStreamCaptureStatusNone)) {
-      if (!o.prp && !pls::make_operand(A, op, o))
-        return pls::exec_fail(A, "matrix format has no GPU SpMM path");
-      if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);
-      const hipError_t e = pls::upload_spmm_form(o, d, tiles());
-      if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM block upload");
-    }
+    if (!o.prp && !pls::make_operand(A, op, o))
+      return pls::exec_fail(A, "matrix format has no GPU SpMM path");
+    // A plan that has a form may get the other one inside a capture (a plan's
+    // first wide product there is left to the capture's own rules): the build's
+    // allocations and copies are no part of the graph.
+    const bool second = d.lb_state == 1 && d.has_form(!tiles());
+    const RelaxedCapture relaxed(second);
+    if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);
+    const hipError_t e = pls::upload_spmm_form(o, d, tiles());
+    if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM block upload");
   }
   if (tiles() && d.has_form(true)) form = pls::SpmmForm::Tiles;
   else if (d.has_form(false)) form = pls::SpmmForm::Lds;

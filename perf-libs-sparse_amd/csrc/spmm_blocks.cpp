@@ -353,18 +353,43 @@ bool cut_clustered(const Operand &o, int32_t umax, const std::vector<int32_t> &c
   return int32_t(h.brow.size()) == m;
 }
 
-// A form's values gathered from the plan's, on a stream of its own and waited
-// for: whichever stream the next product runs on, it finds them written.  (The
-// plan's values themselves are complete: their uploads and updates wait.)
-hipError_t gather_and_wait(VStore vs, void *dst, const DevCsr &d, const DevBuf &epos, int64_t n) {
-  hipStream_t s = nullptr;
-  hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-  if (e != hipSuccess) return e;
-  e = plk::gather_vals(vs, dst, d.vals.get(), epos.as<int32_t>(), n, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipStreamDestroy(s);
-  return e;
-}
+// The copies and the value gather of a form's build, on a stream of their own
+// that is waited for before the form is used: a product on any stream, a captured
+// one too, finds its form written.  (The plan's values themselves are complete:
+// their uploads and updates wait.)
+class BuildStream {
+ public:
+  BuildStream() { e_ = hipStreamCreateWithFlags(&s_, hipStreamNonBlocking); }
+  ~BuildStream() {
+    if (s_) (void)hipStreamDestroy(s_);
+  }
+  BuildStream(const BuildStream &) = delete;
+  BuildStream &operator=(const BuildStream &) = delete;
+  // The host arrays must live until wait().
+  void alloc(DevBuf &dst, size_t bytes) {
+    if (e_ == hipSuccess) e_ = dst.alloc(std::max<size_t>(bytes, 8));
+  }
+  void copy(void *dst, const void *host, size_t bytes) {
+    if (e_ == hipSuccess && bytes) e_ = hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, s_);
+  }
+  template <class T> void upload(DevBuf &dst, const std::vector<T> &host) {
+    alloc(dst, sizeof(T) * host.size());
+    copy(dst.get(), host.data(), sizeof(T) * host.size());
+  }
+  void gather(const DevCsr &d, DevBuf &dst, const DevBuf &epos, int64_t n) {
+    if (e_ == hipSuccess)
+      e_ = plk::gather_vals(d.vs, dst.get(), d.vals.get(), epos.as<int32_t>(), n, s_);
+  }
+  hipError_t wait() {
+    const hipError_t w = s_ ? hipStreamSynchronize(s_) : hipSuccess;
+    if (e_ == hipSuccess) e_ = w;
+    return e_;
+  }
+
+ private:
+  hipStream_t s_ = nullptr;
+  hipError_t e_;
+};
 
 // Clustered blocks also keep their non-zeros in block order: first non-zero
 // of each entry of the row order (prp), list positions, the CSR position of
@@ -374,21 +399,20 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
   d.lb_prp.reset();
   d.lb_epos.reset();
   d.lb_val.reset();
-  hipError_t e =
-      d.lb_ucol.upload(h.ucol.data(), sizeof(int32_t) * std::max<size_t>(h.ucol.size(), 1));
   std::vector<int32_t> prp;  // clustered: first non-zero of each entry of the row order
   // list positions and block-order values end with one padding entry (the
   // kernel stages them in aligned pairs); the CSR plan's values carry theirs
+  const size_t nnz = h.lidx.size();
+  std::vector<int32_t> epos;
+  std::vector<uint8_t> lidx;
   if (h.brow.empty()) {
-    std::vector<uint8_t> lidx(h.lidx);
+    lidx = h.lidx;
     lidx.push_back(0);
-    if (e == hipSuccess) e = d.lb_lidx.upload(lidx.data(), lidx.size());
   } else {
     const int32_t m = o.m, base = o.prp[0];
-    const size_t nnz = h.lidx.size();
     prp.assign(size_t(m) + 1, 0);
-    std::vector<int32_t> epos(nnz + 1, 0);
-    std::vector<uint8_t> lidx(nnz + 1, 0);
+    epos.assign(nnz + 1, 0);
+    lidx.assign(nnz + 1, 0);
     for (int32_t i = 0; i < m; ++i) {
       const int32_t r = h.brow[size_t(i)];
       prp[size_t(i) + 1] = prp[size_t(i)] + (o.prp[r + 1] - o.prp[r]);
@@ -403,15 +427,8 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
         }
       }
     });
-    const size_t es = d.vs == VStore::F64 ? 8 : d.vs == VStore::F32 ? 4 : 2;
-    if (e == hipSuccess) e = d.lb_lidx.upload(lidx.data(), lidx.size());
-    if (e == hipSuccess) e = d.lb_brow.upload(h.brow.data(), sizeof(int32_t) * size_t(m));
-    if (e == hipSuccess) e = d.lb_prp.upload(prp.data(), sizeof(int32_t) * prp.size());
     // the padding entry gathers the CSR plan's own padding value (zero)
     epos[nnz] = int32_t(nnz);
-    if (e == hipSuccess) e = d.lb_epos.upload(epos.data(), sizeof(int32_t) * (nnz + 1));
-    if (e == hipSuccess) e = d.lb_val.alloc(es * (nnz + 1));
-    if (e == hipSuccess) e = gather_and_wait(d.vs, d.lb_val.get(), d, d.lb_epos, int64_t(nnz + 1));
   }
   const auto first = [&](int32_t r) { return h.brow.empty() ? o.prp[r] - o.prp[0] : prp[size_t(r)]; };
   std::vector<SpmmBlock> blocks(h.row0.size() - 1);
@@ -419,8 +436,19 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
     const int32_t r0 = h.row0[b], r1 = h.row0[b + 1], u0 = h.uoff[b];
     blocks[b] = {r0, r1 - r0, u0, h.uoff[b + 1] - u0, first(r0), first(r1) - first(r0)};
   }
-  if (e == hipSuccess)
-    e = d.lb_block.upload(blocks.data(), sizeof(SpmmBlock) * std::max<size_t>(blocks.size(), 1));
+  BuildStream to;
+  to.upload(d.lb_ucol, h.ucol);
+  to.upload(d.lb_lidx, lidx);
+  to.upload(d.lb_block, blocks);
+  if (!h.brow.empty()) {
+    const size_t es = d.vs == VStore::F64 ? 8 : d.vs == VStore::F32 ? 4 : 2;
+    to.upload(d.lb_brow, h.brow);
+    to.upload(d.lb_prp, prp);
+    to.upload(d.lb_epos, epos);
+    to.alloc(d.lb_val, es * (nnz + 1));
+    to.gather(d, d.lb_val, d.lb_epos, int64_t(nnz + 1));
+  }
+  const hipError_t e = to.wait();
   d.lb_lds = e == hipSuccess;
   return e;
 }
@@ -527,16 +555,15 @@ hipError_t upload_tiles(const Operand &o, const LbHost &h, DevCsr &d) {
   end.epos.assign(size_t(kTilePad), int32_t(int64_t(o.prp[o.m]) - base));
   parts.push_back(std::move(end));
   const size_t es = d.vs == VStore::F64 ? 8 : d.vs == VStore::F32 ? 4 : 2;
-  hipError_t e = hipSuccess;
+  BuildStream to;
   auto put = [&](DevBuf &dst, auto member) {
     size_t bytes = 0;
     for (const TileHost &P : parts) bytes += (P.*member).size() * sizeof((P.*member)[0]);
-    if (e == hipSuccess) e = dst.alloc(std::max<size_t>(bytes, 8));
+    to.alloc(dst, bytes);
     size_t at = 0;
     for (const TileHost &P : parts) {
       const size_t n = (P.*member).size() * sizeof((P.*member)[0]);
-      if (e == hipSuccess && n)
-        e = hipMemcpy(static_cast<char *>(dst.get()) + at, (P.*member).data(), n, hipMemcpyHostToDevice);
+      to.copy(static_cast<char *>(dst.get()) + at, (P.*member).data(), n);
       at += n;
     }
   };
@@ -546,10 +573,11 @@ hipError_t upload_tiles(const Operand &o, const LbHost &h, DevCsr &d) {
   put(d.t_col, &TileHost::col);
   put(d.t_epos, &TileHost::epos);
   put(d.t_direct, &TileHost::direct);
-  if (e == hipSuccess) e = d.t_val.alloc(es * (nv + size_t(kTilePad)));
+  to.alloc(d.t_val, es * (nv + size_t(kTilePad)));
   d.t_nnz = int64_t(nv);
   d.t_ndirect = int32_t(nd);
-  if (e == hipSuccess) e = gather_and_wait(d.vs, d.t_val.get(), d, d.t_epos, d.t_nnz + kTilePad);
+  to.gather(d, d.t_val, d.t_epos, d.t_nnz + kTilePad);
+  const hipError_t e = to.wait();
   d.ntiles = e == hipSuccess ? int32_t(nt) : -1;
   return e;
 }

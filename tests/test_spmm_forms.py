@@ -98,3 +98,20 @@ ran = kernels([tuple(x.split()) for x in stub.stub_log().decode().splitlines()])
 assert sum("k_spmm_tile" in f for f in ran) == 100 and sum("k_spmm_lds" in f for f in ran) == 100
 assert sum("k_gather_vals" in f for f in ran) == 1  # the tiles' values
 """)
+
+
+@pytest.mark.parametrize("warm,k,kernel", [(16, 128, "k_spmm_tile"), (128, 16, "k_spmm_lds"), (128, 8, "k_spmm_lds")])
+def test_captured_product_runs_on_the_form_of_its_width(run, warm, k, kernel):
+    """A plan warmed with one width, captured with one of the other form: the
+    form is built beside the capture, with no call that a capture forbids and
+    nothing but the product's kernels on the captured stream."""
+    run(f"""
+product({warm})
+stub.stub_capture(S1)
+calls = product({k}, S1)
+stub.stub_capture(None)
+assert form(calls) == {kernel!r}, calls
+assert not [c for c in calls if c[0] == "unsafe"], calls
+assert all("k_spmm" in c[1] for c in calls if c[0] == "launch" and c[2] == str(S1)), calls
+assert form(product({k}, S1)) == {kernel!r}
+""")
