@@ -180,7 +180,7 @@ perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k, pls::
   auto tiles = [&] { return pls::spmm_on_tiles(d, A->dt == DType::F64, k); };
   const std::lock_guard<std::mutex> lock(d.lb_mutex);
   if (d.lb_state < 0) return PERFLIBS_STATUS_SUCCESS;
-  if (d.lb_state == 0 || !d.has_form(tiles())) {
+  if (d.lb_state == 0 || !(d.has_form(tiles()) || (d.lb_failed && d.has_form(!tiles())))) {
     if (!o.prp && !pls::make_operand(A, op, o))
       return pls::exec_fail(A, "matrix format has no GPU SpMM path");
     // A plan that has a form may get the other one inside a capture (a plan's
@@ -190,10 +190,17 @@ perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k, pls::
     const RelaxedCapture relaxed(second);
     if (d.lb_state == 0) pls::build_spmm_blocks(o, d, A->spmm_rows);
     const hipError_t e = pls::upload_spmm_form(o, d, tiles());
-    if (e != hipSuccess) return pls::hip_fail(A, e, "SpMM block upload");
+    if (e != hipSuccess) {
+      if (!second) return pls::hip_fail(A, e, "SpMM block upload");
+      // no room beside the first form, which then serves every width
+      (void)hipGetLastError();
+      d.lb_failed = true;
+    }
   }
-  if (tiles() && d.has_form(true)) form = pls::SpmmForm::Tiles;
-  else if (d.has_form(false)) form = pls::SpmmForm::Lds;
+  if (d.lb_state == 1) {
+    const bool on_tiles = d.has_form(tiles()) ? tiles() : !tiles();
+    form = on_tiles ? pls::SpmmForm::Tiles : pls::SpmmForm::Lds;
+  }
   return PERFLIBS_STATUS_SUCCESS;
 }
 

@@ -19,6 +19,7 @@ hipError_t DevBuf::alloc(size_t bytes) {
   hipError_t e = hipMalloc(&p_, bytes);
   if (e != hipSuccess) {
     p_ = nullptr;
+    (void)hipGetLastError();  // reported here, not by the next launch's check
     return e;
   }
   bytes_ = bytes;

@@ -154,6 +154,7 @@ struct DevCsr {
   DevBuf lb_val;         // [nnz] vals in block order, storage vs (clustered; refreshed by updates)
   std::shared_ptr<LbHost> lb_host;  // the cut, from which either form below is built on first use
   bool lb_lds = false;              // the arrays above are on the device (k_spmm_lds)
+  bool lb_failed = false;           // no room for a second form: not tried again
   std::mutex lb_mutex;              // held while a form is chosen or built
   // Row tiles of the blocks (k_spmm_tile), on the device when ntiles >= 0
   int32_t ntiles = -1, t_ndirect = 0;

@@ -450,6 +450,9 @@ hipError_t upload_blocks(const Operand &o, const LbHost &h, DevCsr &d) {
   }
   const hipError_t e = to.wait();
   d.lb_lds = e == hipSuccess;
+  if (e != hipSuccess)
+    for (DevBuf *b : {&d.lb_ucol, &d.lb_lidx, &d.lb_block, &d.lb_brow, &d.lb_prp, &d.lb_epos, &d.lb_val})
+      b->reset();
   return e;
 }
 
@@ -579,6 +582,9 @@ hipError_t upload_tiles(const Operand &o, const LbHost &h, DevCsr &d) {
   to.gather(d, d.t_val, d.t_epos, d.t_nnz + kTilePad);
   const hipError_t e = to.wait();
   d.ntiles = e == hipSuccess ? int32_t(nt) : -1;
+  if (e != hipSuccess)
+    for (DevBuf *b : {&d.t_tiles, &d.t_row, &d.t_mask, &d.t_col, &d.t_epos, &d.t_direct, &d.t_val})
+      b->reset();
   return e;
 }
 }  // namespace
@@ -643,7 +649,7 @@ void build_spmm_blocks(const Operand &o, DevCsr &d, int rows) {
   d.lb_ucols = int64_t(h->ucol.size());
   d.lb_umax = umax;
   d.lb_clustered = !h->brow.empty();
-  d.lb_lds = false;
+  d.lb_lds = d.lb_failed = false;
   d.ntiles = -1;
   d.lb_host = used ? std::move(h) : nullptr;
   d.lb_state = used ? 1 : -1;

@@ -103,7 +103,10 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, in
 hipError_t hipMalloc(void **p, size_t n) {
   if (unsafe("hipMalloc")) return hipErrorStreamCaptureUnsupported;
   const std::lock_guard<std::mutex> l(mu);
-  if (live_bytes + n > limit_bytes) return fail(hipErrorOutOfMemory);
+  if (live_bytes + n > limit_bytes) {
+    log_text += "nomem\n";
+    return fail(hipErrorOutOfMemory);
+  }
   *p = std::calloc(1, n);
   sizes[*p] = n;
   live_bytes += n;

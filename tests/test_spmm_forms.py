@@ -115,3 +115,36 @@ assert not [c for c in calls if c[0] == "unsafe"], calls
 assert all("k_spmm" in c[1] for c in calls if c[0] == "launch" and c[2] == str(S1)), calls
 assert form(product({k}, S1)) == {kernel!r}
 """)
+
+
+@pytest.mark.parametrize("warm,k,kernel", [(16, 128, "k_spmm_lds"), (128, 16, "k_spmm_tile")])
+def test_no_room_for_a_second_form(run, warm, k, kernel):
+    """The form that is there serves a product whose own form does not fit, and
+    the build is not tried again by every product after it."""
+    run(f"""
+product({warm})
+held = stub.stub_live()
+stub.stub_limit(held + 1000)
+calls = product({k})
+assert ("nomem",) in calls and form(calls) == {kernel!r}, calls
+assert stub.stub_live() == held  # nothing of the failed build is kept
+assert ("nomem",) not in product({k}) and form(product({warm})) == {kernel!r}
+stub.stub_limit(1 << 40)
+A.set_spmm_rows(1)  # a new cut tries again
+assert form(product({warm})) == {kernel!r} and form(product({k})) != {kernel!r}
+""")
+
+
+def test_no_room_for_the_first_form_is_an_error(run):
+    run("""
+product(4)
+stub.stub_limit(stub.stub_live() + 1000)
+for k in (16, 128):
+    try:
+        product(k)
+    except P.PerflibsError:
+        continue
+    raise AssertionError(k)
+stub.stub_limit(1 << 40)
+assert form(product(128)) == "k_spmm_tile"
+""")
