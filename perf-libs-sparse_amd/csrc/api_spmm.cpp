@@ -195,6 +195,7 @@ perflibs_status_t csr_plan_for(perflibs_spmat_top_t *A, int op, int64_t k, pls::
       // no room beside the first form, which then serves every width
       (void)hipGetLastError();
       d.lb_failed = true;
+      d.lb_host.reset();
     }
   }
   if (d.lb_state == 1) {

@@ -152,7 +152,7 @@ struct DevCsr {
   DevBuf lb_prp;         // int32 [m+1] first non-zero of each entry of the row order (clustered)
   DevBuf lb_epos;        // int32 [nnz] CSR position of each non-zero in block order (clustered)
   DevBuf lb_val;         // [nnz] vals in block order, storage vs (clustered; refreshed by updates)
-  std::shared_ptr<LbHost> lb_host;  // the cut, from which either form below is built on first use
+  std::shared_ptr<LbHost> lb_host;  // the cut, kept until both forms below are built (each on first use)
   bool lb_lds = false;              // the arrays above are on the device (k_spmm_lds)
   bool lb_failed = false;           // no room for a second form: not tried again
   std::mutex lb_mutex;              // held while a form is chosen or built

@@ -657,7 +657,10 @@ void build_spmm_blocks(const Operand &o, DevCsr &d, int rows) {
 
 hipError_t upload_spmm_form(const Operand &o, DevCsr &d, bool tiles) {
   if (d.lb_state != 1 || (tiles ? d.ntiles >= 0 : d.lb_lds)) return hipSuccess;
-  return tiles ? upload_tiles(o, *d.lb_host, d) : upload_blocks(o, *d.lb_host, d);
+  const hipError_t e = tiles ? upload_tiles(o, *d.lb_host, d) : upload_blocks(o, *d.lb_host, d);
+  // the cut (a byte per non-zero, the lists and the row order) until both are there
+  if (d.has_form(true) && d.has_form(false)) d.lb_host.reset();
+  return e;
 }
 
 int spmm_blocks_host(const Operand &o, int rows, int32_t *nblocks, int32_t *list_max,

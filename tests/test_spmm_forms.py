@@ -148,3 +148,27 @@ for k in (16, 128):
 stub.stub_limit(1 << 40)
 assert form(product(128)) == "k_spmm_tile"
 """)
+
+
+def test_the_cut_is_given_back_when_both_forms_exist(run):
+    run("""
+from plsparse import workloads as W
+class Info(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_size_t) for f in "arena ordblks smblks hblks hblkhd usmblks fsmblks uordblks fordblks keepcost".split()]
+libc = ctypes.CDLL(None)
+libc.mallinfo2.restype = Info
+def host():  # heap in use, without the stub's device memory
+    i = libc.mallinfo2()
+    return i.uordblks + i.hblkhd - stub.stub_live()
+rp, ci, v = W.stencil27(60)
+T = P.SpMat.csr(60 ** 3, 60 ** 3, rp, ci, v, flags=P.CREATE_NOCOPY)
+product(4, h=T)
+before = host()
+product(16, h=T)
+assert host() - before > len(v)  # the cut: a byte per non-zero and the lists
+product(128, h=T)
+assert host() - before < len(v) // 4
+assert form(product(16, h=T)) == "k_spmm_lds" and form(product(128, h=T)) == "k_spmm_tile"
+T.set_spmm_rows(1)  # and cut again from the handle's arrays
+assert form(product(16, h=T)) == "k_spmm_lds" and form(product(128, h=T)) == "k_spmm_tile"
+""")
