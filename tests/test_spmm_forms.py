@@ -172,3 +172,20 @@ assert form(product(16, h=T)) == "k_spmm_lds" and form(product(128, h=T)) == "k_
 T.set_spmm_rows(1)  # and cut again from the handle's arrays
 assert form(product(16, h=T)) == "k_spmm_lds" and form(product(128, h=T)) == "k_spmm_tile"
 """)
+
+
+def test_the_narrow_tile_cases_reach_their_kernels(run):
+    run("""
+from test_gpu_spmm_tiles_narrow import CASES, wide_band
+rp, ci, v = wide_band()
+m = len(rp) - 1
+H = {}
+for prec, k, (nw, vw) in CASES:
+    if prec not in H:
+        H[prec] = P.SpMat.csr(m, m, rp, ci, v.astype(np.float32))
+        if prec == "bf16":
+            H[prec].set_precision(P.VALUES_BF16)
+    ran = kernels(product(k, h=H[prec]))
+    want = f"k_spmm_tileILi{nw}ELi{vw}E{'tf' if prec == 'bf16' else 'ff'}"
+    assert any(want in f for f in ran), (prec, k, ran, H[prec].spmm_info())
+""")
