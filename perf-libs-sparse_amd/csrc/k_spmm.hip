@@ -128,6 +128,22 @@ __global__ __launch_bounds__(kBlock) void k_spmm_gather(
   }
 }
 
+// One element of C.
+template <class X, bool BETA>
+__device__ __forceinline__ void store_one(X *c, acc_t<X> v, acc_t<X> alpha, acc_t<X> beta) {
+  acc_t<X> r = alpha * v;
+  if (BETA) r += beta * acc_t<X>(*c);
+  *c = X(r);
+}
+
+// x[i] of an array in registers.
+template <int N> __device__ __forceinline__ int64_t pick(const uint32_t (&x)[N], int32_t i) {
+  uint32_t v = x[0];
+#pragma unroll
+  for (int j = 1; j < N; ++j) v = i == j ? x[j] : v;
+  return v;
+}
+
 // VW columns of one C row from column c0 on; the lane owns those from `own` on.
 template <int VW, class X, bool BETA>
 __device__ __forceinline__ void store_cols(X *crow, int64_t c0, int64_t own, int32_t k,
@@ -158,6 +174,26 @@ __device__ __forceinline__ void store_cols(X *crow, int64_t c0, int64_t own, int
   }
 }
 
+// The same in a wave with a NaN among its results (redo): an element that is NaN
+// is not stored; the returned bits name them.
+template <int VW, class X, bool BETA>
+__device__ __forceinline__ uint32_t store_or_mark(bool redo, X *crow, int64_t c0, int64_t own,
+                                                  int32_t k, const acc_t<X> (&v)[VW],
+                                                  acc_t<X> alpha, acc_t<X> beta) {
+  uint32_t nans = 0;
+  if (!redo) {
+    store_cols<VW, X, BETA>(crow, c0, own, k, v, alpha, beta);
+  } else {
+#pragma unroll
+    for (int e = 0; e < VW; ++e) {
+      if (c0 + e < own) continue;
+      if (v[e] == v[e]) store_one<X, BETA>(crow + c0 + e, v[e], alpha, beta);
+      else nans |= 1u << e;
+    }
+  }
+  return nans;
+}
+
 // Row tiles (pls::spmm_on_tiles: operands whose rows share columns, k > 16): one
 // wave multiplies a tile of up to 32 rows, two halves of 16, by a window of NW *
 // 16 * VW columns of B on the matrix cores.  The tile's distinct columns are
@@ -177,9 +213,13 @@ __device__ __forceinline__ void store_cols(X *crow, int64_t c0, int64_t own, int
 // matrix cores 106), k = 128 on 80^3 408 us (floor 257): matrix cores about half
 // busy and 2.5 GB moved for 1.2 GB, B rows fetched again across grid planes.
 // k_spmm_lds took 275 and 553 us there, with its present staging 497 at k = 128.
-// A wave whose results hold a NaN computes them again entry by entry: a column
-// some row of the tile does not have is multiplied by zero for that row, which
-// changes nothing unless the B value is infinite or NaN.
+// An element that comes out NaN is computed again entry by entry: a column some
+// row of the tile does not have is multiplied by zero for that row, which changes
+// nothing unless the B value is infinite or NaN, and then leaves NaN in that
+// element.  A wave with such elements stores the others, lists these in its LDS
+// slice and takes one per lane, up to the first NaN (27-point 80^3, FP64 k = 32,
+// 122 us: one bad entry 124, a column of NaN 181, of infinities 274, all of B NaN
+// 269; all elements of such waves one after the other 221 / 1488 / 1488 / 1486).
 template <class X> struct TileAcc;
 template <> struct TileAcc<double> {
   typedef double T __attribute__((ext_vector_type(4)));
@@ -196,15 +236,25 @@ template <> struct TileAcc<float> {
   static __device__ __forceinline__ int row(int kk, int r) { return 4 * kk + r; }
 };
 
+// One element of A*B from its entries, four in flight, up to the first NaN.
 template <class V, class X>
-__device__ __noinline__ acc_t<X> csr_dot(int32_t p0, int32_t p1, int64_t c, const int32_t *ci,
-                                         const V *val, const X *Bm, int64_t ldb) {
-  acc_t<X> s = 0;
-  for (int32_t p = p0; p < p1; ++p)
-    s += acc_t<X>(ldv(val, p)) * acc_t<X>(Bm[int64_t(ci[p]) * ldb + c]);
+__device__ __forceinline__ acc_t<X> csr_dot(int32_t p0, int32_t p1, int64_t c, const int32_t *ci,
+                                            const V *val, const X *Bm, int64_t ldb) {
+  using A = acc_t<X>;
+  A s = 0;
+  for (int32_t p = p0; p < p1 && s == s; p += 4) {
+    A a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int32_t q = min(p + u, p1 - 1);
+      a[u] = A(ldv(val, q));
+      b[u] = A(Bm[int64_t(ci[q]) * ldb + c]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s = p + u < p1 ? s + a[u] * b[u] : s;
+  }
   return s;
 }
-
 template <int NW, int VW, class V, class X, bool BETA>
 __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
     int32_t tile0, int32_t ntiles, int32_t win0, int32_t k, const pls::SpmmTile *__restrict__ tiles,
@@ -225,11 +275,12 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
   if (tile >= ntiles) return;
   const int32_t pass = win0 + int32_t(blockIdx.y);
   const pls::SpmmTile t0 = tiles[tile], t1 = tiles[tile + 1];
-  int64_t own[NW], c0[NW];
+  uint32_t own[NW];  // below 2^31 + a window
+  int32_t c0[NW];    // -1 where a window of one column (k = 1) is the rest of a wider B
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    own[w] = (int64_t(pass) * NW + w) * (16 * VW) + n * VW;
-    c0[w] = min(own[w], int64_t(k - VW));
+    own[w] = (uint32_t(pass) * NW + w) * (16 * VW) + n * VW;
+    c0[w] = int32_t(min(int64_t(own[w]), int64_t(k - VW)));
   }
   typename M::T acc[2][NW][VW];
 #pragma unroll
@@ -294,6 +345,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
       __builtin_amdgcn_wave_barrier();
     }
   }
+  const int32_t nrows = t1.row0 - t0.row0;
   bool nan = false;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -304,7 +356,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
 #pragma unroll
         for (int r = 0; r < 4; ++r) nan = nan || acc[h][w][e][r] != acc[h][w][e][r];
   const bool redo = __any(nan);
-  const int32_t nrows = t1.row0 - t0.row0;
+  uint64_t nans = 0;  // the lane's elements to be computed again
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -317,12 +369,37 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
         A out[VW];
 #pragma unroll
         for (int e = 0; e < VW; ++e) out[e] = acc[h][w][e][r];
-        if (redo)
-          for (int e = 0; e < VW; ++e)
-            out[e] = csr_dot<V, X>(rp[row], rp[row + 1], c0[w] + e, ci, val, Bm, ldb);
-        store_cols<VW, X, BETA>(Cm + int64_t(row) * ldc, c0[w], own[w], k, out, alpha, beta);
+        nans |= uint64_t(store_or_mark<VW, X, BETA>(redo, Cm + int64_t(row) * ldc, c0[w], own[w], k,
+                                                    out, alpha, beta))
+                << (((h * 4 + r) * NW + w) * VW);
       }
     }
+  if (!redo) return;
+  // listed in the wave's LDS slice as lane + 64 * element, a lane for each
+  constexpr int CAP = sizeof(A) * G * 128 / 4, NE = 8 * NW * VW;
+  uint32_t *list = reinterpret_cast<uint32_t *>(av);
+  int32_t cnt = 0;
+  for (int32_t s = 0; s < NE; ++s) {
+    const bool mine = nans >> s & 1;
+    const uint64_t all = __ballot(mine);
+    if (mine)
+      list[cnt + int32_t(__builtin_amdgcn_mbcnt_hi(
+                     uint32_t(all >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(all), 0)))] =
+          uint32_t(lane + 64 * s);
+    cnt += __builtin_popcountll(all);
+    if (s + 1 < NE && cnt + 64 <= CAP) continue;
+    __builtin_amdgcn_wave_barrier();
+    for (int32_t j = lane; j < cnt; j += 64) {
+      const int32_t l = int32_t(list[j] & 63u), el = int32_t(list[j] >> 6);
+      const int32_t e = el % VW, w = el / VW % NW, r = el / (VW * NW) & 3, h = el / (VW * NW * 4);
+      const int32_t row = trow[t0.row0 + M::row(l >> 4, r) + (h ? t0.half : 0)];
+      const int64_t c = min((int64_t(pass) * NW + w) * (16 * VW) + (l & 15) * VW, int64_t(k - VW)) + e;
+      store_one<X, BETA>(Cm + int64_t(row) * ldc + c,
+                         csr_dot<V, X>(rp[row], rp[row + 1], c, ci, val, Bm, ldb), alpha, beta);
+    }
+    __builtin_amdgcn_wave_barrier();
+    cnt = 0;
+  }
 }
 
 // Column-compressed row blocks (k >= 8 when the plan's block lists are short
@@ -678,18 +755,27 @@ __global__ __launch_bounds__(kBlock) void k_csr_few_rhs(
 // A stored zero adds nothing, as in the zero-dropped CSR product of the
 // reference (src/matmul.cpp:619-649), even against an infinite or NaN B value.
 // The tiles do multiply stored zeros: 0 * finite adds a zero, which changes
-// nothing, and 0 * Inf or 0 * NaN makes the accumulator NaN.  So a wave whose
-// results hold a NaN computes them again entry by entry, skipping zeros.
+// nothing, and 0 * Inf or 0 * NaN makes the accumulator NaN.  So an element that
+// comes out NaN is computed again entry by entry, skipping zeros, up to the first
+// NaN, after the wave has stored its others (8 x 8 24^3, FP64 k = 8, 40 us: a
+// column of NaN 48, all of B NaN 56; with all elements of such waves computed
+// again to their last entry 1812 and 1809).
 template <int BS, bool CM, class V, class X>
-__device__ __noinline__ acc_t<X> bsr_dot_nonzero(int32_t p0, int32_t p1, int32_t r, int64_t c,
-                                                 const int32_t *ci, const V *val, const X *Bm,
-                                                 int64_t ldb) {
+__device__ __forceinline__ acc_t<X> bsr_dot_nonzero(int32_t p0, int32_t p1, int32_t r, int64_t c,
+                                                    const int32_t *ci, const V *val, const X *Bm,
+                                                    int64_t ldb) {
   acc_t<X> s = 0;
-  for (int32_t p = p0; p < p1; ++p)
-    for (int32_t j = 0; j < BS; ++j) {
-      const acc_t<X> a = acc_t<X>(ldv(val, int64_t(p) * (BS * BS) + (CM ? j * BS + r : r * BS + j)));
-      if (a != acc_t<X>(0)) s += a * acc_t<X>(Bm[(int64_t(ci[p]) * BS + j) * ldb + c]);
+  for (int32_t p = p0; p < p1 && s == s; ++p) {  // up to the first NaN
+    acc_t<X> a[BS], b[BS];
+    const X *Bc = Bm + int64_t(ci[p]) * BS * ldb + c;
+#pragma unroll
+    for (int j = 0; j < BS; ++j) {
+      a[j] = acc_t<X>(ldv(val, int64_t(p) * (BS * BS) + (CM ? j * BS + r : r * BS + j)));
+      b[j] = acc_t<X>(Bc[j * ldb]);
     }
+#pragma unroll
+    for (int j = 0; j < BS; ++j) s = a[j] != acc_t<X>(0) ? s + a[j] * b[j] : s;
+  }
   return s;
 }
 
@@ -768,11 +854,11 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f64(
   const int32_t pass = int32_t(unit % npass);
   const int n = lane & 3, nb = (lane >> 2) % NB, pb = ((lane >> 2) & 3) / NB, kk = lane >> 4;
   const int32_t br = int32_t(unit / npass) * (ROWS ? PB * R : 1) + (ROWS ? pb : 0);
-  int64_t own[NW], c0[NW];
+  uint32_t own[NW], c0[NW];  // below 2^31 + a window
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    own[w] = (int64_t(pass) * NW + w) * (4 * NB * VW) + (nb * 4 + n) * VW;
-    c0[w] = min(own[w], int64_t(k - VW));
+    own[w] = (uint32_t(pass) * NW + w) * (4 * NB * VW) + (nb * 4 + n) * VW;
+    c0[w] = min(own[w], uint32_t(k - VW));
   }
   int32_t p0[R], p1[R], steps = 0;
   double acc[R][T][NW][VW];
@@ -854,24 +940,30 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f64(
           nan = nan || acc[i][it][w][e] != acc[i][it][w][e];
         }
   const bool redo = __any(nan);
+  uint32_t nans = 0;  // the lane's elements to be computed again
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    if (br + i * PB >= mb) return;
+    if (br + i * PB >= mb || !(ROWS || pb == 0)) continue;
 #pragma unroll
     for (int it = 0; it < T; ++it) {
       const int32_t r = T == 2 ? (CM ? 2 * kk + it : it * 4 + kk) : kk;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        if (redo)
-          for (int e = 0; e < VW; ++e)
-            acc[i][it][w][e] = bsr_dot_nonzero<BS, CM, double, double>(p0[i], p1[i], r, c0[w] + e,
-                                                                       ci, val, Bm, ldb);
-        if (ROWS || pb == 0)
-          store_cols<VW, double, BETA>(Cm + (int64_t(br + i * PB) * BS + r) * ldc, c0[w], own[w],
-                                       k, acc[i][it][w], alpha, beta);
-      }
+      for (int w = 0; w < NW; ++w)
+        nans |= store_or_mark<VW, double, BETA>(redo, Cm + (int64_t(br + i * PB) * BS + r) * ldc,
+                                                c0[w], own[w], k, acc[i][it][w], alpha, beta)
+                << (((i * T + it) * NW + w) * VW);
     }
   }
+  if (!redo) return;
+  for (int32_t s = 0; s < R * T * NW * VW; ++s)
+    if (nans >> s & 1) {
+      const int32_t e = s % VW, w = s / VW % NW, it = s / (VW * NW) % T, row = br + s / (VW * NW * T) * PB;
+      const int32_t r = T == 2 ? (CM ? 2 * kk + it : it * 4 + kk) : kk;
+      const int64_t c = pick(c0, w) + e;
+      store_one<double, BETA>(Cm + (int64_t(row) * BS + r) * ldc + c,
+                              bsr_dot_nonzero<BS, CM, double, double>(rp[row], rp[row + 1], r, c, ci, val, Bm, ldb),
+                              alpha, beta);
+    }
 }
 
 // FP32 (and BF16 values): lane = n + 4 * (nb + NB * (kk + KL * pb)) holds
@@ -896,11 +988,11 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f32(
   const int32_t pass = int32_t(unit % npass);
   const int n = lane & 3, nb = (lane >> 2) % NB, g = (lane >> 2) / NB, kk = g % KL, pb = g / KL;
   const int32_t br = int32_t(unit / npass) * (ROWS ? PB : 1) + (ROWS ? pb : 0);
-  int64_t own[NW], c0[NW];
+  uint32_t own[NW], c0[NW];  // below 2^31 + a window
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    own[w] = (int64_t(pass) * NW + w) * (4 * NB * VW) + (nb * 4 + n) * VW;
-    c0[w] = min(own[w], int64_t(k - VW));
+    own[w] = (uint32_t(pass) * NW + w) * (4 * NB * VW) + (nb * 4 + n) * VW;
+    c0[w] = min(own[w], uint32_t(k - VW));
   }
   const bool live = br < mb;
   const int32_t p0 = live ? rp[br] : 0, p1 = live ? rp[br + 1] : 0;
@@ -978,6 +1070,7 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f32(
         }
     const bool redo = __any(nan);
     if (!live) return;
+    uint32_t nans = 0;  // the lane's elements to be computed again
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = CM ? T * i + kk : kk * 4 + i;
@@ -986,13 +1079,19 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f32(
         float out[VW];
 #pragma unroll
         for (int e = 0; e < VW; ++e) out[e] = acc[0][w][e][i];
-        if (redo)
-          for (int e = 0; e < VW; ++e)
-            out[e] = bsr_dot_nonzero<BS, CM, V, float>(p0, p1, r, c0[w] + e, ci, val, Bm, ldb);
-        store_cols<VW, float, BETA>(Cm + (int64_t(br) * BS + r) * ldc, c0[w], own[w], k, out,
-                                    alpha, beta);
+        nans |= store_or_mark<VW, float, BETA>(redo, Cm + (int64_t(br) * BS + r) * ldc, c0[w], own[w],
+                                               k, out, alpha, beta)
+                << ((i * NW + w) * VW);
       }
     }
+    if (!redo) return;
+    for (int32_t s = 0; s < 4 * NW * VW; ++s)
+      if (nans >> s & 1) {
+        const int32_t e = s % VW, w = s / VW % NW, i = s / (VW * NW), r = CM ? T * i + kk : kk * 4 + i;
+        const int64_t c = pick(c0, w) + e;
+        store_one<float, BETA>(Cm + (int64_t(br) * BS + r) * ldc + c,
+                               bsr_dot_nonzero<BS, CM, V, float>(p0, p1, r, c, ci, val, Bm, ldb), alpha, beta);
+      }
     return;
   }
   // sum over the lanes g = (kk, pb): at each of the low bits a lane keeps half
@@ -1021,15 +1120,21 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f32(
     }
   const bool redo = __any(nan);
   const int gr = g % BS, r = CM ? T * (gr % 4) + gr / 4 : gr;  // the lane's block row
+  if (g >= BS) return;
+  uint32_t nans = 0;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    if (redo)
-      for (int e = 0; e < VW; ++e)
-        out[w][e] = bsr_dot_nonzero<BS, CM, V, float>(p0, p1, r, c0[w] + e, ci, val, Bm, ldb);
-    if (g < BS)
-      store_cols<VW, float, BETA>(Cm + (int64_t(br) * BS + r) * ldc, c0[w], own[w], k, out[w],
-                                  alpha, beta);
-  }
+  for (int w = 0; w < NW; ++w)
+    nans |= store_or_mark<VW, float, BETA>(redo, Cm + (int64_t(br) * BS + r) * ldc, c0[w], own[w], k,
+                                           out[w], alpha, beta)
+            << (w * VW);
+  if (!redo) return;
+  for (int32_t s = 0; s < NW * VW; ++s)
+    if (nans >> s & 1) {
+      const int32_t e = s % VW, w = s / VW;
+      const int64_t c = pick(c0, w) + e;
+      store_one<float, BETA>(Cm + (int64_t(br) * BS + r) * ldc + c,
+                             bsr_dot_nonzero<BS, CM, V, float>(p0, p1, r, c, ci, val, Bm, ldb), alpha, beta);
+    }
 }
 
 template <class X>
