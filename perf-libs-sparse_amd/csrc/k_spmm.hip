@@ -199,7 +199,8 @@ __device__ __forceinline__ uint32_t store_or_mark(bool redo, X *crow, int64_t c0
 // 16 * VW columns of B on the matrix cores.  The tile's distinct columns are
 // listed four to a step; a step's B rows are read once, VW adjacent columns per
 // lane (the columns of a window are permuted), and serve both halves through
-// v_mfma_f64_16x16x4 / v_mfma_f32_16x16x4.  The values stay compressed: per step
+// v_mfma_f64_16x16x4 / v_mfma_f32_16x16x4.  alpha is multiplied into the values, as
+// in the other CSR kernels.  The values stay compressed: per step
 // and half the non-zero ones in lane order behind a 64-bit mask of the lanes
 // that have one.  They are copied to the wave's LDS slice with full-width loads
 // one group of G steps ahead, and each lane picks its own by counting mask bits
@@ -236,10 +237,11 @@ template <> struct TileAcc<float> {
   static __device__ __forceinline__ int row(int kk, int r) { return 4 * kk + r; }
 };
 
-// One element of A*B from its entries, four in flight, up to the first NaN.
+// One element of alpha*A*B from its entries, four in flight, up to the first NaN.
 template <class V, class X>
-__device__ __forceinline__ acc_t<X> csr_dot(int32_t p0, int32_t p1, int64_t c, const int32_t *ci,
-                                            const V *val, const X *Bm, int64_t ldb) {
+__device__ __forceinline__ acc_t<X> csr_dot(acc_t<X> alpha, int32_t p0, int32_t p1, int64_t c,
+                                            const int32_t *ci, const V *val, const X *Bm,
+                                            int64_t ldb) {
   using A = acc_t<X>;
   A s = 0;
   for (int32_t p = p0; p < p1 && s == s; p += 4) {
@@ -247,7 +249,7 @@ __device__ __forceinline__ acc_t<X> csr_dot(int32_t p0, int32_t p1, int64_t c, c
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int32_t q = min(p + u, p1 - 1);
-      a[u] = A(ldv(val, q));
+      a[u] = alpha * A(ldv(val, q));
       b[u] = A(Bm[int64_t(ci[q]) * ldb + c]);
     }
 #pragma unroll
@@ -321,8 +323,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
           nv += __builtin_popcountll(m[u][h]);
         }
 #pragma unroll
-      for (int i = 0; i < PF; ++i) av[lane + 64 * i] = pf[i];
-      for (int32_t i = 64 * PF; i < nv; i += 64) av[lane + i] = A(ldv(tv, lane + i));
+      for (int i = 0; i < PF; ++i) av[lane + 64 * i] = alpha * pf[i];
+      for (int32_t i = 64 * PF; i < nv; i += 64) av[lane + i] = alpha * A(ldv(tv, lane + i));
       tv += nv;
 #pragma unroll
       for (int i = 0; i < PF; ++i) pf[i] = A(ldv(tv, lane + 64 * i));
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
 #pragma unroll
         for (int e = 0; e < VW; ++e) out[e] = acc[h][w][e][r];
         nans |= uint64_t(store_or_mark<VW, X, BETA>(redo, Cm + int64_t(row) * ldc, c0[w], own[w], k,
-                                                    out, alpha, beta))
+                                                    out, A(1), beta))
                 << (((h * 4 + r) * NW + w) * VW);
       }
     }
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_tile(
       const int32_t row = trow[t0.row0 + M::row(l >> 4, r) + (h ? t0.half : 0)];
       const int64_t c = min((int64_t(pass) * NW + w) * (16 * VW) + (l & 15) * VW, int64_t(k - VW)) + e;
       store_one<X, BETA>(Cm + int64_t(row) * ldc + c,
-                         csr_dot<V, X>(rp[row], rp[row + 1], c, ci, val, Bm, ldb), alpha, beta);
+                         csr_dot<V, X>(alpha, rp[row], rp[row + 1], c, ci, val, Bm, ldb), A(1), beta);
     }
     __builtin_amdgcn_wave_barrier();
     cnt = 0;
