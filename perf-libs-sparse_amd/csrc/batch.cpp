@@ -13,11 +13,12 @@
 // sell_structure): a chunk table, columns, values and a slot -> row map, built
 // on the host from the device copy of those problems.
 //
-// exec launches one kernel over all CSR tiles (and one over the SELL-C-sigma
-// tiles) from a hipGraph captured once per (alpha, beta, shape).  optimize(autotune) times candidate tile sizes,
-// per-k-class row shapes (lanes per row, columns per lane) and the SELL-C-sigma
-// (C, sigma) of the k = 1 problems by graph replays on scratch outputs and
-// keeps the fastest, one coordinate at a time.
+// exec launches one kernel over all CSR tiles (and, when there are many of them,
+// one over the SELL-C-sigma tiles) from a hipGraph captured once per (alpha,
+// beta, shape).  optimize(autotune) times candidate tile sizes, per-k-class row
+// shapes (lanes per row, columns per lane) and the SELL-C-sigma (C, sigma) of the
+// k = 1 problems by graph replays on scratch outputs and keeps the fastest, one
+// coordinate at a time.
 #include <algorithm>
 #include <atomic>
 #include <climits>
@@ -175,6 +176,7 @@ plk::BatchLaunch launch_of(const perflibs_amd_batch_s *B, const void *xs, const 
   L.ntiles = B->ntiles;
   L.ncsr = B->ncsr;
   L.grid = B->grid;
+  L.resident = B->cus * B->occ;
   L.tiles = B->tiles_d.as<BatchTile>();
   L.rp = B->rp.as<int32_t>();
   L.ci = B->ci.as<int32_t>();

@@ -43,6 +43,14 @@ template <class A> struct BatchRegs {
   int32_t r[NR];
 };
 
+// SELL-C-sigma arrays of the batch.
+template <class V> struct BatchSell {
+  const BatchSellChunk *chunks;
+  const int32_t *ci;
+  const V *val;
+  const int32_t *perm;
+};
+
 template <class A> __device__ __forceinline__ bool batch_staged(const BatchTile &tl) {
   return tl.nnz <= kBatchStage && tl.nrows <= kBatchRows<A>;
 }
@@ -170,27 +178,26 @@ __device__ __forceinline__ void batch_rows(const BatchTile &tl, int G,
 // column / value slices of a chunk are contiguous across its lanes, so each
 // step of the row loop is one coalesced load per array; padding slots hold
 // value 0 and column 0 of the problem.  Four non-zeros in flight per lane.
-// A kernel of its own, launched after the CSR tiles': it needs no LDS and a
-// quarter of their registers (256 banded problems, all k = 1, C = 32: FP64 /
+// Many of them run in a kernel of their own after the CSR tiles': it needs no LDS
+// and a quarter of their registers (256 banded problems, all k = 1, C = 32: FP64 /
 // FP32 379 / 297 us as tiles of one kernel, 261 / 192 on its own; the two
 // launches as parallel branches of the graph took 615 us where one after the
-// other take 496).
+// other take 496).  Few of them run beside the CSR tiles (batch_sell_beside).
 template <int C, class V, class X, bool BETA>
-__global__ __launch_bounds__(kBlock) void k_batch_sell(
-    const BatchTile *__restrict__ tiles, const BatchSellChunk *__restrict__ chunks,
-    const int32_t *__restrict__ sci, const V *__restrict__ sval, const int32_t *__restrict__ perm,
-    const X *const *__restrict__ xs, X *const *__restrict__ ys, acc_t<X> alpha, acc_t<X> beta) {
+__device__ __forceinline__ void batch_sell(const BatchTile &tl, const BatchSell<V> &sell,
+                                           const X *const *__restrict__ xs,
+                                           X *const *__restrict__ ys, acc_t<X> alpha,
+                                           acc_t<X> beta) {
   using A = acc_t<X>;
-  const BatchTile tl = tiles[blockIdx.x];
   const X *xp = xs[tl.prob];
   X *yp = ys[tl.prob];
   const int tid = threadIdx.x, r = tid % C;
   for (int32_t c = tl.r0 + tid / C; c < tl.r1; c += kBlock / C) {
-    const BatchSellChunk ch = chunks[c];
+    const BatchSellChunk ch = sell.chunks[c];
     A acc = 0;
     if (alpha != A(0)) {
-      const int32_t *cc = sci + ch.off + r;
-      const V *vv = sval + ch.off + r;
+      const int32_t *cc = sell.ci + ch.off + r;
+      const V *vv = sell.val + ch.off + r;
       int32_t j = 0;
       for (; j + 4 <= ch.width; j += 4) {
         int32_t col[4];
@@ -205,7 +212,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_sell(
       }
       for (; j < ch.width; ++j) acc += A(ldv(vv, int64_t(j) * C)) * A(xp[ldi(cc, int64_t(j) * C)]);
     }
-    const int32_t row = perm[ch.slot0 + r];
+    const int32_t row = sell.perm[ch.slot0 + r];
     if (row >= 0) {
       A res = alpha * acc;
       if (BETA) res += beta * A(yp[row]);
@@ -213,29 +220,42 @@ __global__ __launch_bounds__(kBlock) void k_batch_sell(
     }
   }
 }
+template <int C, class V, class X, bool BETA>
+__global__ __launch_bounds__(kBlock) void k_batch_sell(const BatchTile *__restrict__ tiles,
+                                                       BatchSell<V> sell,
+                                                       const X *const *__restrict__ xs,
+                                                       X *const *__restrict__ ys, acc_t<X> alpha,
+                                                       acc_t<X> beta) {
+  batch_sell<C, V, X, BETA>(tiles[blockIdx.x], sell, xs, ys, alpha, beta);
+}
 
 // A workgroup has its next tile's record, entries and row offsets on their way
 // (in registers) while it computes the current one from LDS: a tile then waits
 // for its X rows only (256 banded problems, FP64 / FP32: 508 / 317 -> 495 / 295
 // us).  That takes 125 VGPRs in FP64, so four workgroups share a CU; five or six
 // spill and take 792 / 952 us.
-template <class V, class X, bool BETA>
+template <int SELLC, class V, class X, bool BETA>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_batch(
     int32_t ntiles, const BatchTile *__restrict__ tiles, const int32_t *__restrict__ rp_all,
     const int32_t *__restrict__ ci_all, const V *__restrict__ val_all,
     const X *const *__restrict__ xs, X *const *__restrict__ ys, acc_t<X> alpha, acc_t<X> beta,
-    BatchShape shape) {
+    BatchShape shape, int32_t grid, BatchSell<V> sell) {
   using A = acc_t<X>;
   __shared__ BatchLds<A> lds;
   BatchRegs<A> g;
   int32_t t = blockIdx.x;
+  if constexpr (SELLC > 0)  // the workgroups past the CSR tiles' grid: a SELL tile each
+    if (t >= grid) {
+      batch_sell<SELLC, V, X, BETA>(tiles[ntiles + t - grid], sell, xs, ys, alpha, beta);
+      return;
+    }
   if (t >= ntiles) return;
   BatchTile tl = tiles[t];
   const X *xp = xs[tl.prob];
   X *yp = ys[tl.prob];
   batch_load(tl, rp_all, ci_all, val_all, g);
   for (;;) {
-    const int32_t nt = t + gridDim.x;
+    const int32_t nt = t + grid;
     const bool more = nt < ntiles;
     BatchTile next = tl;
     if (more) next = tiles[nt];
@@ -275,6 +295,22 @@ template <class F> hipError_t batch_types(pls::VStore vs, bool dbl, F &&f) {
 }
 }  // namespace
 
+// Whether the SELL-C-sigma tiles share the CSR tiles' launch.  Beside them they fill
+// the CUs that the persistent workgroups leave, and there is one launch, but four
+// workgroups to a CU; after them there are eight.  The line is a few rounds of the
+// chip, farther out for C = 64 (half the loads per row in a wave), which gains
+// only where most tiles are SELL (banded problems, k = 1, 4, 16 mixed, tile 2048,
+// FP64 us beside / after: C = 32, 16 / 32 / 48 / 256 problems 30 / 49 / 76 / 479
+// against 38 / 57 / 73 / 471; C = 64 29 / 47 / 69 / 453 against 38 / 55 / 76 / 478;
+// 7 of 8 problems k = 1, C = 32 26 / 41 / 69 / 409 against 32 / 40 / 61 / 312, C =
+// 64 23 / 34 / 57 / 346 against 31 / 43 / 65 / 336).
+static bool batch_sell_beside(const BatchLaunch &L) {
+  const int64_t nsell = L.ntiles - L.ncsr;
+  if (nsell <= 0 || L.ncsr <= 0) return false;
+  return L.sell_C == 32 ? nsell <= 3 * int64_t(L.resident)
+                        : nsell <= 6 * int64_t(L.resident) || nsell <= L.ncsr;
+}
+
 hipError_t batch_launch(const BatchLaunch &L, hipStream_t s) {
   if (L.ntiles == 0 || L.grid == 0) return hipSuccess;
   return batch_types(L.vs, L.dbl, [&](auto vtag, auto xtag) -> hipError_t {
@@ -284,18 +320,24 @@ hipError_t batch_launch(const BatchLaunch &L, hipStream_t s) {
     auto *ys = static_cast<X *const *>(L.ys);
     const auto *sv = static_cast<const V *>(L.svals);
     const auto *tiles = L.tiles;
-    auto csr = [&](auto kern) {
-      kern<<<std::min(L.grid, L.ncsr), kBlock, 0, s>>>(
-          L.ncsr, tiles, L.rp, L.ci, static_cast<const V *>(L.vals), xs, ys, acc_t<X>(L.alpha),
-          acc_t<X>(L.beta), L.shape);
+    const BatchSell<V> sl{L.chunks, L.sci, sv, L.perm};
+    const bool upd = L.beta != 0.0;
+    const int32_t grid = std::min(L.grid, L.ncsr), nsell = L.ntiles - L.ncsr;
+    auto csr = [&](auto kern, int32_t more) {
+      kern<<<grid + more, kBlock, 0, s>>>(L.ncsr, tiles, L.rp, L.ci, static_cast<const V *>(L.vals), xs,
+                                          ys, acc_t<X>(L.alpha), acc_t<X>(L.beta), L.shape, grid, sl);
     };
     auto sell = [&](auto kern) {
-      kern<<<L.ntiles - L.ncsr, kBlock, 0, s>>>(tiles + L.ncsr, L.chunks, L.sci, sv, L.perm, xs, ys,
-                                                acc_t<X>(L.alpha), acc_t<X>(L.beta));
+      kern<<<nsell, kBlock, 0, s>>>(tiles + L.ncsr, sl, xs, ys, acc_t<X>(L.alpha),
+                                    acc_t<X>(L.beta));
     };
-    const bool upd = L.beta != 0.0;
-    if (L.ncsr > 0) upd ? csr(k_batch<V, X, true>) : csr(k_batch<V, X, false>);
-    if (L.ntiles > L.ncsr) {
+    if (batch_sell_beside(L)) {
+      if (L.sell_C == 32) upd ? csr(k_batch<32, V, X, true>, nsell) : csr(k_batch<32, V, X, false>, nsell);
+      else upd ? csr(k_batch<64, V, X, true>, nsell) : csr(k_batch<64, V, X, false>, nsell);
+      return hipGetLastError();
+    }
+    if (L.ncsr > 0) upd ? csr(k_batch<0, V, X, true>, 0) : csr(k_batch<0, V, X, false>, 0);
+    if (nsell > 0) {
       if (L.sell_C == 32) upd ? sell(k_batch_sell<32, V, X, true>) : sell(k_batch_sell<32, V, X, false>);
       else upd ? sell(k_batch_sell<64, V, X, true>) : sell(k_batch_sell<64, V, X, false>);
     }
@@ -308,7 +350,7 @@ int batch_occupancy(bool dbl, pls::VStore vs) {
   hipError_t e = batch_types(vs, dbl, [&](auto vtag, auto xtag) -> hipError_t {
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
-    const void *kern = reinterpret_cast<const void *>(&k_batch<V, X, false>);
+    const void *kern = reinterpret_cast<const void *>(&k_batch<0, V, X, false>);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, kBlock, 0);
   });
   return e == hipSuccess ? nb : 0;

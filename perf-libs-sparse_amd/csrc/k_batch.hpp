@@ -59,6 +59,7 @@ struct BatchLaunch {
   bool dbl = true;
   pls::VStore vs = pls::VStore::F64;
   int32_t ntiles = 0, ncsr = 0, grid = 0;  // the first ncsr tiles are CSR, the rest SELL-C-sigma
+  int32_t resident = 0;                    // workgroups of the CSR kernel the device holds at once
   const BatchTile *tiles = nullptr;
   const int32_t *rp = nullptr, *ci = nullptr;
   const void *vals = nullptr;

@@ -70,8 +70,8 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
   *s = config.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t s) {
-  note("launch " + names[f] + " " + id(s));
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3, void **, size_t, hipStream_t s) {
+  note("launch " + names[f] + " " + id(s) + " " + std::to_string(grid.x));
   return hipSuccess;
 }
 hipError_t hipGetDeviceCount(int *n) {
@@ -154,6 +154,18 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st) {
   *st = capturing && s == capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) {
+  *g = nullptr;
+  return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
+  *e = nullptr;
+  return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m) {
   std::swap(*m, mode);
   return hipSuccess;

@@ -189,3 +189,33 @@ for prec, k, (nw, vw) in CASES:
     want = f"k_spmm_tileILi{nw}ELi{vw}E{'tf' if prec == 'bf16' else 'ff'}"
     assert any(want in f for f in ran), (prec, k, ran, H[prec].spmm_info())
 """)
+
+
+def test_sell_tiles_of_a_batch_beside_or_after_the_csr_tiles(run):
+    """Few SELL tiles share the CSR tiles' launch; many get their own after it."""
+    run("""
+from plsparse import workloads as W
+from test_gpu_batch_loop import CASES, problems
+seen = set()
+for kind, tile, C, sigma in CASES:
+    probs = problems(W, kind)
+    mats = [P.SpMat.csr(p[0], p[0], p[1], p[2], p[3]) for p in probs]
+    B = P.Batch(mats, [p[4] for p in probs])
+    B.set_shape(tile, [2, 2, 2, 8, 8], [1, 1, 2, 1, 2])
+    if C:
+        B.set_sell(C, sigma)
+    ptr = [buf.ctypes.data] * len(probs)
+    B.set_operands(ptr, ptr)
+    stub.stub_clear()
+    B.exec(0.75, 0.5)
+    ran = [(c[1], int(c[3])) for c in (x.split() for x in stub.stub_log().decode().splitlines()) if c[0] == "launch"]
+    resident, tiles = 256 * 4, B.info()["ntiles"]
+    if C == 0:
+        assert len(ran) == 1 and "k_batchILi0E" in ran[0][0] and ran[0][1] == min(tiles, resident), ran
+    elif len(ran) == 1:  # beside
+        assert f"k_batchILi{C}E" in ran[0][0], ran
+    else:
+        assert "k_batchILi0E" in ran[0][0] and f"k_batch_sellILi{C}E" in ran[1][0] and ran[1][1] > 3 * resident, ran
+    seen.add((C, len(ran), tiles > resident))
+assert {(32, 1, False), (32, 2, True), (64, 1, True), (64, 2, True), (0, 1, True)} <= seen, seen
+""")
