@@ -1,12 +1,12 @@
-// k_batch.hip — a persistent launch over a batch of independent CSR
+// k_batch.hip — one launch over a batch of independent CSR
 // products Y_p = alpha * A_p * X_p + beta * Y_p (X_p: n_p x k_p, Y_p: m_p x k_p,
 // row-major; k_p = 1 is SpMV).
 //
 // The host cuts every problem into row tiles of bounded nnz and sorts the
 // tiles by estimated cost, largest first; workgroup b takes tiles b, b + G,
-// b + 2G, ... (G = resident workgroups), a static greedy schedule that needs
-// no queue counter, so the launch can be captured in a hipGraph and replayed
-// as is.  Inside a tile a row is handled by a group of `lanes` lanes (a power
+// b + 2G, ... (G = resident workgroups; one tile each when the device holds them
+// all at once), a static greedy schedule that needs no queue counter, so the
+// launch can be captured in a hipGraph and replayed as is.  Inside a tile a row is handled by a group of `lanes` lanes (a power
 // of two): the k_p right-hand-side columns are split over k_p / cpl lanes (cpl
 // consecutive columns per lane, read as one contiguous piece of the X row),
 // and the row's non-zeros over the remaining lanes / (k_p / cpl) subsets,
@@ -229,13 +229,17 @@ __global__ __launch_bounds__(kBlock) void k_batch_sell(const BatchTile *__restri
   batch_sell<C, V, X, BETA>(tiles[blockIdx.x], sell, xs, ys, alpha, beta);
 }
 
-// A workgroup has its next tile's record, entries and row offsets on their way
-// (in registers) while it computes the current one from LDS: a tile then waits
-// for its X rows only (256 banded problems, FP64 / FP32: 508 / 317 -> 495 / 295
-// us).  That takes 125 VGPRs in FP64, so four workgroups share a CU; five or six
-// spill and take 792 / 952 us.
-template <int SELLC, class V, class X, bool BETA>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_batch(
+// LOOP: a persistent workgroup has its next tile's record, entries and row
+// offsets on their way (in registers) while it computes the current one from LDS:
+// a tile then waits for its X rows only (256 banded problems, FP64 / FP32: 508 /
+// 317 -> 495 / 295 us).  That takes 125 VGPRs in FP64, so four workgroups share a
+// CU; five or six spill and take 792 / 952 us.  Without LOOP each has one tile and
+// six share a CU: for batches that then run all at once, 1.5 times what the
+// persistent ones hold (16 / 12 problems, 1,424 / 1,299 tiles, k = 16, FP32 27.1 ->
+// 22.9 / 26.3 -> 21.9 us, FP64, 8 problems, 1,180 tiles, 36.5 -> 33.2; at 2,109
+// tiles it is 33.0 -> 34.4).
+template <int SELLC, bool LOOP, class V, class X, bool BETA>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(LOOP ? 4 : 6))) void k_batch(
     int32_t ntiles, const BatchTile *__restrict__ tiles, const int32_t *__restrict__ rp_all,
     const int32_t *__restrict__ ci_all, const V *__restrict__ val_all,
     const X *const *__restrict__ xs, X *const *__restrict__ ys, acc_t<X> alpha, acc_t<X> beta,
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
   batch_load(tl, rp_all, ci_all, val_all, g);
   for (;;) {
     const int32_t nt = t + grid;
-    const bool more = nt < ntiles;
+    const bool more = LOOP && nt < ntiles;
     BatchTile next = tl;
     if (more) next = tiles[nt];
     __syncthreads();  // the previous tile is done with the LDS
@@ -322,22 +326,29 @@ hipError_t batch_launch(const BatchLaunch &L, hipStream_t s) {
     const auto *tiles = L.tiles;
     const BatchSell<V> sl{L.chunks, L.sci, sv, L.perm};
     const bool upd = L.beta != 0.0;
-    const int32_t grid = std::min(L.grid, L.ncsr), nsell = L.ntiles - L.ncsr;
-    auto csr = [&](auto kern, int32_t more) {
-      kern<<<grid + more, kBlock, 0, s>>>(L.ncsr, tiles, L.rp, L.ci, static_cast<const V *>(L.vals), xs,
-                                          ys, acc_t<X>(L.alpha), acc_t<X>(L.beta), L.shape, grid, sl);
+    const bool loop = 2 * int64_t(L.ncsr) > 3 * int64_t(L.resident);
+    const int32_t grid = loop ? std::min(L.grid, L.ncsr) : L.ncsr, nsell = L.ntiles - L.ncsr;
+    auto with = [&](auto sell_c, auto lp, int32_t more) {
+      constexpr int C = decltype(sell_c)::value;
+      constexpr bool LOOP = decltype(lp)::value;
+      auto go = [&](auto kern) {
+        kern<<<grid + more, kBlock, 0, s>>>(L.ncsr, tiles, L.rp, L.ci, static_cast<const V *>(L.vals),
+                                            xs, ys, acc_t<X>(L.alpha), acc_t<X>(L.beta), L.shape, grid, sl);
+      };
+      upd ? go(k_batch<C, LOOP, V, X, true>) : go(k_batch<C, LOOP, V, X, false>);
+    };
+    auto csr = [&](auto sell_c, int32_t more) {
+      loop ? with(sell_c, std::true_type{}, more) : with(sell_c, std::false_type{}, more);
     };
     auto sell = [&](auto kern) {
       kern<<<nsell, kBlock, 0, s>>>(tiles + L.ncsr, sl, xs, ys, acc_t<X>(L.alpha),
                                     acc_t<X>(L.beta));
     };
-    if (batch_sell_beside(L)) {
-      if (L.sell_C == 32) upd ? csr(k_batch<32, V, X, true>, nsell) : csr(k_batch<32, V, X, false>, nsell);
-      else upd ? csr(k_batch<64, V, X, true>, nsell) : csr(k_batch<64, V, X, false>, nsell);
-      return hipGetLastError();
-    }
-    if (L.ncsr > 0) upd ? csr(k_batch<0, V, X, true>, 0) : csr(k_batch<0, V, X, false>, 0);
-    if (nsell > 0) {
+    const bool beside = batch_sell_beside(L);
+    if (beside && L.sell_C == 32) csr(std::integral_constant<int, 32>{}, nsell);
+    else if (beside) csr(std::integral_constant<int, 64>{}, nsell);
+    else if (L.ncsr > 0) csr(std::integral_constant<int, 0>{}, 0);
+    if (nsell > 0 && !beside) {
       if (L.sell_C == 32) upd ? sell(k_batch_sell<32, V, X, true>) : sell(k_batch_sell<32, V, X, false>);
       else upd ? sell(k_batch_sell<64, V, X, true>) : sell(k_batch_sell<64, V, X, false>);
     }
@@ -350,7 +361,7 @@ int batch_occupancy(bool dbl, pls::VStore vs) {
   hipError_t e = batch_types(vs, dbl, [&](auto vtag, auto xtag) -> hipError_t {
     using V = std::remove_const_t<std::remove_pointer_t<decltype(vtag)>>;
     using X = std::remove_pointer_t<decltype(xtag)>;
-    const void *kern = reinterpret_cast<const void *>(&k_batch<0, V, X, false>);
+    const void *kern = reinterpret_cast<const void *>(&k_batch<0, true, V, X, false>);
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, kBlock, 0);
   });
   return e == hipSuccess ? nb : 0;

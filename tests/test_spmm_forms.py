@@ -211,7 +211,9 @@ for kind, tile, C, sigma in CASES:
     ran = [(c[1], int(c[3])) for c in (x.split() for x in stub.stub_log().decode().splitlines()) if c[0] == "launch"]
     resident, tiles = 256 * 4, B.info()["ntiles"]
     if C == 0:
-        assert len(ran) == 1 and "k_batchILi0E" in ran[0][0] and ran[0][1] == min(tiles, resident), ran
+        loop = tiles > 1.5 * resident
+        assert len(ran) == 1 and f"k_batchILi0ELb{int(loop)}" in ran[0][0], ran
+        assert ran[0][1] == (resident if loop else tiles), ran
     elif len(ran) == 1:  # beside
         assert f"k_batchILi{C}E" in ran[0][0], ran
     else:
