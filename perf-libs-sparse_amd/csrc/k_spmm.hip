@@ -748,7 +748,7 @@ __global__ __launch_bounds__(kBlock) void k_csr_few_rhs(
 // costs nothing).  No LDS and few registers: occupancy hides the latency.
 // Bound: the block stream and the B rows re-fetched across grid planes.  27
 // blocks per row, 8 x 8, block grid 32^3, FP64 k = 8 / 32 / 128: 94 / 168 / 483
-// us (4.9 TB/s at k = 8); FP32 61 / 88 / 301.  Scalar FMAs on a b x CPL register
+// us (4.9 TB/s at k = 8); FP32 37 / 89 / 284.  Scalar FMAs on a b x CPL register
 // tile, with the block broadcast from LDS and a select per product for stored
 // zeros, took 151 / 292 / 993 and 103 / 159 / 500.
 // Loads need element alignment only; a lane that would run past column k
@@ -781,19 +781,29 @@ __device__ __forceinline__ acc_t<X> bsr_dot_nonzero(int32_t p0, int32_t p1, int3
   return s;
 }
 
-// N adjacent block values (1, 2, 4; aligned to their size) as one load.
+// Block values, kept in the caches: several loads share a line (the rows or
+// columns of a block, neighbouring block rows of a wave), and one that is not kept
+// is fetched again for each (us non-temporal / kept, k = 8: 4 x 4, 9 per row, FP32
+// column-major 58 / 23, row-major 33 / 22, FP64 51 / 39; 8 x 8 block grid 32^3 FP32
+// 61 / 37).  FP64 blocks are streamed past them in windows of 64 columns and more,
+// where the B rows need the room (8 x 8, 7 per row, k = 64 92 / 97), and when they
+// are more than the MALL holds (k = 8, 8 x 8 269 MB 64 / 54, 405 MB 91 / 95, 4 x 4
+// 349 MB 96 / 99; column-major 8 x 8 blocks, of which a load takes single columns,
+// 405 MB 110 / 96), and where few blocks share a row (k = 32, 8 x 8, 3 per row 50 /
+// 54, 4 x 4, 7 per row 79 / 83; block-diagonal 4 x 4, k = 24 54 / 60).
+template <bool KEEP, class T> __device__ __forceinline__ T ld_block(const T *p) {
+  if constexpr (KEEP) return *p;
+  else return __builtin_nontemporal_load(p);
+}
+// N adjacent ones (1, 2, 4; aligned to their size) as one load.
 template <int N, class V>
 __device__ __forceinline__ void ld_adjacent(const V *p, float (&x)[N]) {
-  if constexpr (N == 1) {
-    x[0] = ldv(p, 0);
-  } else {
-    typedef V VN __attribute__((ext_vector_type(N)));
-    const VN t = __builtin_nontemporal_load(reinterpret_cast<const VN *>(p));
+  typedef V VN __attribute__((ext_vector_type(N)));
+  const VN t = ld_block<true>(reinterpret_cast<const VN *>(p));
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      if constexpr (sizeof(V) == 2) x[i] = __uint_as_float(uint32_t(V(t[i])) << 16);
-      else x[i] = t[i];
-    }
+  for (int i = 0; i < N; ++i) {
+    if constexpr (sizeof(V) == 2) x[i] = __uint_as_float(uint32_t(V(t[i])) << 16);
+    else x[i] = t[i];
   }
 }
 
@@ -839,7 +849,7 @@ __device__ __forceinline__ BsrAt bsr_at(int32_t s, int32_t u, int32_t pb, int32_
 // Block rows per lane of the short-row FP64 kernel.
 template <int BS, int NW> constexpr int bsr_rows_f64 = BS == 8 ? 1 : NW == 1 ? 4 : 2;
 
-template <int BS, int NB, int NW, int VW, bool ROWS, bool CM, bool BETA>
+template <int BS, int NB, int NW, int VW, bool ROWS, bool CM, bool KEEP, bool BETA>
 __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f64(
     int64_t unit0, int64_t units, int32_t npass, int32_t mb, int32_t k, const int32_t *__restrict__ rp,
     const int32_t *__restrict__ ci, const double *__restrict__ val, const double *__restrict__ Bm,
@@ -896,13 +906,13 @@ __global__ __launch_bounds__(kBlock) void k_bsr_mfma_f64(
         if constexpr (T == 2) {
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
-            const D2 x = __builtin_nontemporal_load(reinterpret_cast<const D2 *>(
+            const D2 x = ld_block<KEEP>(reinterpret_cast<const D2 *>(
                 v + (CM ? (2 * kk + t) * BS + 2 * n : (t * 4 + n) * BS + 2 * kk)));
             a[u][CM ? 0 : t][CM ? t : 0] = on ? x.x : 0.0;
             a[u][CM ? 1 : t][CM ? t : 1] = on ? x.y : 0.0;
           }
         } else {
-          const double x = ldv(v, CM ? kk * BS + n : n * BS + kk);
+          const double x = ld_block<KEEP>(v + (CM ? kk * BS + n : n * BS + kk));
           a[u][0][0] = on ? x : 0.0;
         }
 #pragma unroll
@@ -1392,8 +1402,11 @@ void launch_bsr_mfma(const pls::DevBsr &A, int32_t k, double alpha, const void *
   };
   auto by_type = [&](auto ctag, auto btag) {
     constexpr bool CM = decltype(ctag)::value, BETA = decltype(btag)::value;
-    if constexpr (sizeof(X) == 8) go(k_bsr_mfma_f64<BS, NB, NW, VW, ROWS, CM, BETA>);
-    else go(k_bsr_mfma_f32<BS, NB, NW, BS / 4, VW, ROWS, CM, V, BETA>);
+    if constexpr (sizeof(X) == 4) go(k_bsr_mfma_f32<BS, NB, NW, BS / 4, VW, ROWS, CM, V, BETA>);
+    else if (WCOLS <= 32 && A.nnzb >= (WCOLS <= 16 ? 2 : 8) * int64_t(A.mb) &&
+             (A.vals.bytes() <= size_t(288) << 20 || (BS == 8 && CM)))  // see ld_block
+      go(k_bsr_mfma_f64<BS, NB, NW, VW, ROWS, CM, WCOLS <= 32, BETA>);
+    else go(k_bsr_mfma_f64<BS, NB, NW, VW, ROWS, CM, false, BETA>);
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
@@ -1409,11 +1422,15 @@ void dispatch_bsr_spmm(const pls::DevBsr &A, int32_t k, double alpha, const void
   // x 1-4, e.g. 8 x 8 FP64 k = 32 as NB x NW 4 x 1 / 2 x 2 / 1 x 4: 186 / 168 /
   // 193 us, k = 128 in windows of 32 / 64 / 128: 612 / 525 / 486.  FP32 lanes
   // per block row KL = BS / 4 (16-byte block loads), k = 32 with KL = 8 / 4 / 2:
-  // 143 / 99 / 92; two windows per wave at k = 64 measured 189 against 172.
+  // 143 / 99 / 92; two windows per wave at k = 64 measured 189 against 172 (all
+  // with non-temporal block loads, before ld_block).  Few columns take 1 or 2 per
+  // lane, so that no lane repeats another's (4 x 4, 9 per row, FP32 k = 4 / 7 in
+  // windows of 16: 33 / 45 us, of 4 and 8: 29 / 37), and short 4 x 4 block rows at
+  // k = 9 to 16 two column tiles (46 / 40 at k = 9).
   auto go = [&](auto rtag) {
     constexpr bool R = decltype(rtag)::value;
     if constexpr (sizeof(X) == 8) {
-      if (k < 2) launch_bsr_mfma<BS, 1, 1, 1, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+      if (k <= 4) launch_bsr_mfma<BS, 1, 1, 1, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       else if (k <= 8) launch_bsr_mfma<BS, 1, 1, 2, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       else if (k <= 16) launch_bsr_mfma<BS, 1, 2, 2, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       else if (k <= 32) launch_bsr_mfma<BS, 2, 2, 2, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
@@ -1421,7 +1438,10 @@ void dispatch_bsr_spmm(const pls::DevBsr &A, int32_t k, double alpha, const void
         launch_bsr_mfma<BS, 2, 4, 2, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       else launch_bsr_mfma<BS, 4, 4, 2, false, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
     } else {
-      if (k < 4) launch_bsr_mfma<BS, 1, 1, 1, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+      if (k <= 4) launch_bsr_mfma<BS, 1, 1, 1, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+      else if (k <= 8) launch_bsr_mfma<BS, 1, 1, 2, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
+      else if (k <= 16 && BS == 4 && R)
+        launch_bsr_mfma<BS, 2, 1, 2, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       else if (k <= 16) launch_bsr_mfma<BS, 1, 1, 4, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
       else if (k <= 32 || BS == 8)
         launch_bsr_mfma<BS, 2, 1, 4, R, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
@@ -1429,11 +1449,18 @@ void dispatch_bsr_spmm(const pls::DevBsr &A, int32_t k, double alpha, const void
     }
   };
   // Short block rows: one lane group per block row instead of several sharing
-  // one (block-diagonal 4 x 4, 400,000 block rows, FP64 k = 8: 130 -> 36 us; at
-  // 8 / 12 blocks per row 21 / 20 us against 21 / 22, 8 x 8 at 5 / 8 blocks 17 /
-  // 13 against 13 / 14; 4 x 4 FP32 with its 16 or more lane groups, k = 8: 20
-  // against 15 at 10 blocks, k = 64 40 against 48).
-  const int32_t few = BS == 8 ? 6 : sizeof(X) == 4 && k <= 16 ? 12 : 9;
+  // one, where there are rows enough for that (a wave takes 4 to 16 of them).  Mean
+  // lengths below which it is faster, by block rows (us shared / own, k = 8): 4 x 4
+  // FP64 60,000 rows, 12 blocks per row 28.5 / 22.6, 50,000, 16 25.0 / 26.5; 20,000,
+  // 9 11.4 / 10.1, 12 11.9 / 13.5; 8,000, 4 4.7 / 4.9, 7 5.1 / 6.0.  FP32 60,000, 12
+  // 22.5 / 14.9, 20,000, 12 8.2 / 7.4; 8,000, 7 5.3 / 5.1, 9 4.7 / 5.6.  8 x 8 FP64
+  // 20,000, 5 15.1 / 12.4; 30,000, 7 21.6 / 24.1; 2,000, 3 5.4 / 5.3, 5 4.9 / 5.8.
+  // FP32 20,000, 12 15.5 / 14.9, 15,000, 16 13.4 / 16.2; 8,000, 7 5.8 / 5.8, 12 7.1 /
+  // 7.6; 2,000, 4 5.2 / 5.2, 9 5.0 / 6.1.
+  const int32_t mb = A.mb;
+  const int32_t few = BS == 4 ? (sizeof(X) == 8 ? (mb >= 49152 ? 13 : mb >= 16384 ? 10 : 5)
+                                                : (mb >= 16384 ? 13 : 7))
+                      : mb < 4096 ? 4 : sizeof(X) == 8 ? 6 : mb >= 16384 ? 12 : 8;
   if (A.nnzb < int64_t(A.mb) * few) go(std::true_type{});
   else go(std::false_type{});
 }

@@ -221,3 +221,21 @@ for kind, tile, C, sigma in CASES:
     seen.add((C, len(ran), tiles > resident))
 assert {(32, 1, False), (32, 2, True), (64, 1, True), (64, 2, True), (0, 1, True)} <= seen, seen
 """)
+
+
+def test_block_row_lengths_choose_the_block_kernel(run):
+    run("""
+from plsparse import workloads as W
+from test_gpu_bsr_spmm_rows import CASES
+for mb, b, per, prec, own in CASES:
+    rp, ci, v = W.block_random(mb, b, per, 300, 5)
+    H = P.SpMat.bsr(P.ROW_MAJOR, mb * b, mb * b, b, rp, ci, v.astype(np.float64 if prec == "f64" else np.float32),
+                    flags=P.CREATE_NOCOPY)
+    if prec == "bf16":
+        H.set_precision(P.VALUES_BF16)
+    for k, window in ((3, "ELi1"), (8, "ELi2")):
+        f = kernels(product(k, h=H))[-1]
+        kl = "" if prec == "f64" else f"ELi{b // 4}"
+        assert f"Li{b}ELi1ELi1{kl}{window}ELb{int(own)}E" in f, (mb, b, per, prec, k, f)
+    H.destroy()
+""")
