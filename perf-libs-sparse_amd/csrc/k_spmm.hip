@@ -1248,7 +1248,7 @@ void dispatch_tile(const pls::DevCsr &A, int32_t k, double alpha, const void *B,
     // (27-point 80^3, k = 65 / 96 391 / 380 -> 339 / 344 us, banded 200k rows 234 /
     // 227 -> 205 / 201), unless a second launch of so few tiles costs more (28^3
     // k = 65 25 -> 32).  Its lanes may read columns of the windows before it.
-    const int32_t c = k > 64 && k % 64 <= 32 && A.lb_ucols >= 320000 ? k / 64 * 64 : k;
+    const int32_t c = k > 64 && pls::spmm_tile_cols(A, true, k) % 64 != 0 ? k / 64 * 64 : k;
     if (k <= 32) launch_tile<1, 2, V, X>(A, k, alpha, B, ldb, beta, C, ldc, s);
     else launch_tile<2, 2, V, X>(A, c, alpha, B, ldb, beta, C, ldc, s);
     if (c < k)

@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <memory>
 #include <mutex>
@@ -184,22 +185,53 @@ constexpr int32_t kLbUcolsLarge = 256;
 constexpr int32_t lb_nnz_per_ucol(int32_t umax) { return umax > kLbUcolsSmall ? 8 : 7; }
 constexpr int32_t kLbRows = 128;
 
+// Columns of B that the windows of k_spmm_tile take for k of them.  An FP64 rest of
+// up to 32 behind windows of 64 gets a window of 32 where there are lists enough for
+// its launch.
+inline int64_t spmm_tile_cols(const DevCsr &d, bool dbl, int64_t k) {
+  if (!dbl) return k <= 32 ? 32 : k <= 64 ? 64 : (k + 127) / 128 * 128;
+  if (k <= 32) return 32;
+  return k > 64 && k % 64 <= 32 && d.lb_ucols >= 320000 ? (k + 31) / 32 * 32 : (k + 63) / 64 * 64;
+}
 // Whether a product with k columns runs on the row tiles (k_spmm_tile) or
 // stages the blocks' B rows in LDS (k_spmm_lds).  Tiles read a B row about as
-// often but need no barriers, and multiply on the matrix cores (27-point
-// stencil 80^3, LDS against tiles, FP64 k = 32 / 64 / 128: 157 / 282 / 497 against
-// 122 / 217 / 407 us, FP32 k = 64 / 128 138 / 239 against 118 / 215).  LDS is
-// faster for k <= 16 (half of a 32-column product idle: FP64 k = 16 82 against 106
-// us), for FP32 of up to 32 columns, one LDS chunk, unless rows are long (27-point
-// 80^3 / 64^3, 27 non-zeros per row, k = 32: 69 / 40 against 79 / 48; 4 x 4 and
-// 8 x 8 block stencils, 108 and 216 per row: 37 and 38 against 32 and 30), for
-// short rows (5-point 500^2, FP64 k = 32: 27 against 36 us: too few steps per
-// tile) and for operands with too few steps to hide a tile's latency (27-point
-// 28^3, 114k listed columns, FP64 k = 32 / 48: 11.6 / 16.2 against 13.2 / 18.2 us;
-// 36^3, 242k: 19.4 / 26.4 against 18.9 / 26.9).
+// often but need no barriers, and multiply on the matrix cores; what they take per
+// column of their windows against a column of the LDS chunks (`cost`) falls with the
+// length of a row (us on LDS / tiles, 27-point stencil 80^3, 26 non-zeros per row:
+// FP64 k = 32 / 64 / 128 136 / 117, 256 / 210, 495 / 411, FP32 k = 64 / 128 114 / 109,
+// 219 / 213; 4 x 4 block stencil 24^3, 99 per row, k = 64 FP64 133 / 65, FP32 55 / 41;
+// band of 100, 11 per row, k = 64 FP64 31 / 47, FP32 18 / 28).  Windows wider than k
+// count in full (80^3 FP32 k = 96 / 160 168 / 199, 268 / 378; band of 200, 200,000
+// rows, FP64 k = 24 in LDS chunks of 8 56 / 73).
+// FP32 of up to 32 columns, one LDS chunk, stays in LDS unless rows are long (80^3 64
+// / 74; 8 x 8 block stencil 16^3 36 / 28), and so do FP64 rows of under 20 up to 128
+// columns (16 per row, 100,000 rows, k = 96 88 on tiles, 79 on the slower staging of
+// before).  Fewer tiles than waves that fit hide less of each other's latency (FP32,
+// 16 per row, k = 128, 100,000 rows 57 on tiles, 50 on that staging; 400,000 rows, k =
+// 100 181 / 169).
+// Up to 160,000 listed columns a tile's latency is all there is and its windows run
+// side by side, so there k decides (28^3, 106k, FP64 k = 48 / 96 15 / 18, 27 / 24;
+// FP32 k = 96 / 160 16 / 18, 26 / 25; 36^3, 213k, FP64 k = 32 18 / 18) and, for FP32 of
+// 65 to 96, whether tiles list few columns (band of 50, 3,000 rows, 2.2 per row, k =
+// 96 14 / 13; 14^3, 4.2 per row, 12 / 16).
 inline bool spmm_on_tiles(const DevCsr &d, bool dbl, int64_t k) {
-  return d.lb_state == 1 && k > 16 && d.nnz >= (dbl || k > 32 ? 10 : 64) * int64_t(d.m) &&
-         (k > 64 || d.lb_ucols >= (dbl || k > 32 ? 160000 : 320000));
+  if (d.lb_state != 1 || k <= 16 || d.nnz < 10 * int64_t(d.m)) return false;
+  const double per = double(d.nnz) / d.m;
+  if (d.lb_ucols < 160000) {
+    const bool few = per >= 16 && (d.lb_ucols <= 3 * int64_t(d.m) || d.lb_ucols > 120000);
+    return k > (dbl || few ? 64 : 96);
+  }
+  const int64_t cols = spmm_tile_cols(d, dbl, k);
+  if (dbl) {
+    const bool large = d.lb_umax > kLbUcolsSmall;
+    const int64_t chunk = large ? 8 : 16;  // LDS columns at a time
+    const double cost = large ? 0.4 + 12 / per : 0.33 + 11.5 / per;
+    return (per >= 20 || k > 128) && cost * double(cols) <= 1.18 * double((k + chunk - 1) / chunk * chunk);
+  }
+  if (k <= 32) return per >= 64 && d.lb_ucols >= 320000;
+  const bool filled = d.m * std::max<int64_t>(1, cols / 128) >= 110000;
+  const double cost = (0.45 + 11 / per) * (filled ? 1.0 : 1.1);
+  return cost * double(cols) <= 1.15 * double((k + 31) / 32 * 32);
 }
 
 // Device SELL-C-sigma (layout of src/sell_c_sigma.hpp:43-104, NOTRANS).
