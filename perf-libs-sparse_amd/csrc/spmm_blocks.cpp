@@ -19,6 +19,10 @@
 // A clustered block's rows are listed in `brow` (the kernel reads them from
 // there); consecutive blocks leave it empty.
 #include <algorithm>
+#include <exception>
+#include <mutex>
+#include <new>
+#include <system_error>
 #include <thread>
 
 #include "plsparse.hpp"
@@ -44,14 +48,31 @@ template <class F> void parallel_ranges(int64_t n, int64_t min_per_range, int64_
     fn(0, int64_t(0), n);
     return;
   }
+  // an exception on a thread (no memory) is the caller's, not the program's end
   std::vector<std::thread> th;
+  std::exception_ptr error;
+  std::mutex mu;
+  auto run = [&](int t, int64_t lo, int64_t hi) {
+    try {
+      fn(t, lo, hi);
+    } catch (...) {
+      const std::lock_guard<std::mutex> lock(mu);
+      error = std::current_exception();
+    }
+  };
+  th.reserve(size_t(nt));
   const int64_t step = (n + nt - 1) / nt;
   for (int64_t t = 0; t < nt; ++t) {
     const int64_t lo = t * step, hi = std::min(n, lo + step);
     if (lo >= hi) break;
-    th.emplace_back([&fn, t, lo, hi] { fn(int(t), lo, hi); });
+    try {
+      th.emplace_back(run, int(t), lo, hi);
+    } catch (const std::system_error &) {  // no further thread: this one does it
+      run(int(t), lo, hi);
+    }
   }
   for (auto &t : th) t.join();
+  if (error) std::rethrow_exception(error);
 }
 
 // Greedy cut of consecutive rows into blocks of at most umax distinct
@@ -657,7 +678,12 @@ void build_spmm_blocks(const Operand &o, DevCsr &d, int rows) {
 
 hipError_t upload_spmm_form(const Operand &o, DevCsr &d, bool tiles) {
   if (d.lb_state != 1 || (tiles ? d.ntiles >= 0 : d.lb_lds)) return hipSuccess;
-  const hipError_t e = tiles ? upload_tiles(o, *d.lb_host, d) : upload_blocks(o, *d.lb_host, d);
+  hipError_t e;
+  try {
+    e = tiles ? upload_tiles(o, *d.lb_host, d) : upload_blocks(o, *d.lb_host, d);
+  } catch (const std::bad_alloc &) {  // host memory: as on the device
+    e = hipErrorOutOfMemory;
+  }
   // the cut (a byte per non-zero, the lists and the row order) until both are there
   if (d.has_form(true) && d.has_form(false)) d.lb_host.reset();
   return e;

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 
 namespace {
@@ -42,7 +43,18 @@ bool unsafe(const char *what) {
 }
 }  // namespace
 
+// Host allocations of at least this many bytes fail.
+static size_t host_limit = SIZE_MAX;
+void *operator new(size_t n) {
+  if (n >= host_limit) throw std::bad_alloc();
+  if (void *p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
 extern "C" {
+void stub_host_limit(size_t bytes) { host_limit = bytes; }
 const char *stub_log() { return log_text.c_str(); }
 void stub_clear() { log_text.clear(); }
 void stub_limit(size_t bytes) { limit_bytes = bytes; }

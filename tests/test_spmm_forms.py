@@ -18,6 +18,7 @@ stub = ctypes.CDLL(None)
 stub.stub_log.restype = ctypes.c_char_p
 stub.stub_live.restype = ctypes.c_size_t
 stub.stub_limit.argtypes = [ctypes.c_size_t]
+stub.stub_host_limit.argtypes = [ctypes.c_size_t]
 stub.stub_capture.argtypes = [ctypes.c_void_p]
 import numpy as np
 import plsparse as P
@@ -238,4 +239,21 @@ for mb, b, per, prec, own in CASES:
         kl = "" if prec == "f64" else f"ELi{b // 4}"
         assert f"Li{b}ELi1ELi1{kl}{window}ELb{int(own)}E" in f, (mb, b, per, prec, k, f)
     H.destroy()
+""")
+
+
+@pytest.mark.parametrize("warm,k,kernel", [(16, 128, "k_spmm_lds"), (128, 16, "k_spmm_tile")])
+def test_no_host_memory_for_a_second_form(run, warm, k, kernel):
+    """An allocation that fails while a form is built, on a thread of the build
+    too, does not end the program."""
+    run(f"""
+from plsparse import workloads as W
+rp, ci, v = W.stencil27(40)
+T = P.SpMat.csr(40 ** 3, 40 ** 3, rp, ci, v, flags=P.CREATE_NOCOPY)
+T.set_spmm_rows(2)
+product({warm}, h=T)
+stub.stub_host_limit(100000)
+assert form(product({k}, h=T)) == {kernel!r}
+stub.stub_host_limit(1 << 60)
+assert form(product({k}, h=T)) == {kernel!r} and form(product({warm}, h=T)) == {kernel!r}
 """)
