@@ -302,17 +302,18 @@ template <class F> hipError_t batch_types(pls::VStore vs, bool dbl, F &&f) {
 // Whether the SELL-C-sigma tiles share the CSR tiles' launch.  Beside them they fill
 // the CUs that the persistent workgroups leave, and there is one launch, but four
 // workgroups to a CU; after them there are eight.  The line is a few rounds of the
-// chip, farther out for C = 64 (half the loads per row in a wave), which gains
-// only where most tiles are SELL (banded problems, k = 1, 4, 16 mixed, tile 2048,
-// FP64 us beside / after: C = 32, 16 / 32 / 48 / 256 problems 30 / 49 / 76 / 479
-// against 38 / 57 / 73 / 471; C = 64 29 / 47 / 69 / 453 against 38 / 55 / 76 / 478;
-// 7 of 8 problems k = 1, C = 32 26 / 41 / 69 / 409 against 32 / 40 / 61 / 312, C =
-// 64 23 / 34 / 57 / 346 against 31 / 43 / 65 / 336).
+// chip, farther out for C = 64 (half the loads per row in a wave) unless most tiles
+// are SELL (banded problems, k = 1, 4, 16 mixed, tile 2048, us beside / after: FP64, C
+// = 32, 16 / 32 / 48 / 256 problems 30 / 49 / 76 / 479 against 38 / 57 / 73 / 471; C =
+// 64 29 / 47 / 69 / 453 against 38 / 55 / 76 / 478; 7 of 8 problems k = 1, C = 32 26 /
+// 41 / 69 / 409 against 32 / 40 / 61 / 312, C = 64 23 / 34 / 57 / 346 against 31 / 43 /
+// 65 / 336; BF16, C = 64, 256 problems 262 against 261, 4096 4160 against 3830).
 static bool batch_sell_beside(const BatchLaunch &L) {
   const int64_t nsell = L.ntiles - L.ncsr;
   if (nsell <= 0 || L.ncsr <= 0) return false;
   return L.sell_C == 32 ? nsell <= 3 * int64_t(L.resident)
-                        : nsell <= 6 * int64_t(L.resident) || nsell <= L.ncsr;
+                        : nsell <= 6 * int64_t(L.resident) ||
+                              (nsell <= L.ncsr && nsell <= 16 * int64_t(L.resident));
 }
 
 hipError_t batch_launch(const BatchLaunch &L, hipStream_t s) {
