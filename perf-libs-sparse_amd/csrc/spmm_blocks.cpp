@@ -374,15 +374,21 @@ bool cut_clustered(const Operand &o, int32_t umax, const std::vector<int32_t> &c
   return int32_t(h.brow.size()) == m;
 }
 
-// The copies and the value gather of a form's build, on a stream of their own
-// that is waited for before the form is used: a product on any stream, a captured
-// one too, finds its form written.  (The plan's values themselves are complete:
-// their uploads and updates wait.)
+// The copies and the value gather of a form's build, waited for before the form is
+// used: a product on any stream finds its form written.  (The plan's values
+// themselves are complete: their uploads and updates wait.)  They run on the library
+// stream, or, while that is being captured, on one of their own (making one takes
+// about as long as the build of a small plan).
 class BuildStream {
  public:
-  BuildStream() { e_ = hipStreamCreateWithFlags(&s_, hipStreamNonBlocking); }
+  BuildStream() : s_(stream()) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    own_ = hipStreamIsCapturing(s_, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+    if (own_) e_ = hipStreamCreateWithFlags(&s_, hipStreamNonBlocking);
+    if (e_ != hipSuccess) s_ = nullptr;
+  }
   ~BuildStream() {
-    if (s_) (void)hipStreamDestroy(s_);
+    if (own_ && s_) (void)hipStreamDestroy(s_);
   }
   BuildStream(const BuildStream &) = delete;
   BuildStream &operator=(const BuildStream &) = delete;
@@ -402,14 +408,15 @@ class BuildStream {
       e_ = plk::gather_vals(d.vs, dst.get(), d.vals.get(), epos.as<int32_t>(), n, s_);
   }
   hipError_t wait() {
-    const hipError_t w = s_ ? hipStreamSynchronize(s_) : hipSuccess;
+    const hipError_t w = own_ && !s_ ? hipSuccess : hipStreamSynchronize(s_);
     if (e_ == hipSuccess) e_ = w;
     return e_;
   }
 
  private:
-  hipStream_t s_ = nullptr;
-  hipError_t e_;
+  hipStream_t s_;
+  bool own_;
+  hipError_t e_ = hipSuccess;
 };
 
 // Clustered blocks also keep their non-zeros in block order: first non-zero
