@@ -231,8 +231,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_sell(const BatchTile *__restri
 
 // LOOP: a persistent workgroup has its next tile's record, entries and row
 // offsets on their way (in registers) while it computes the current one from LDS:
-// a tile then waits for its X rows only (256 banded problems, FP64 / FP32: 508 /
-// 317 -> 495 / 295 us).  That takes 125 VGPRs in FP64, so four workgroups share a
+// a tile then waits for its X rows only (256 banded problems, FP64 / FP32: 546 /
+// 317 -> 505 / 295 us).  That takes 125 VGPRs in FP64, so four workgroups share a
 // CU; five or six spill and take 792 / 952 us.  Without LOOP each has one tile and
 // six share a CU: for batches that then run all at once, 1.5 times what the
 // persistent ones hold (16 / 12 problems, 1,424 / 1,299 tiles, k = 16, FP32 27.1 ->
