@@ -6,14 +6,14 @@
 // tiles by estimated cost, largest first; workgroup b takes tiles b, b + G,
 // b + 2G, ... (G = resident workgroups; one tile each when the device holds them
 // all at once), a static greedy schedule that needs no queue counter, so the
-// launch can be captured in a hipGraph and replayed as is.  Inside a tile a row is handled by a group of `lanes` lanes (a power
-// of two): the k_p right-hand-side columns are split over k_p / cpl lanes (cpl
-// consecutive columns per lane, read as one contiguous piece of the X row),
-// and the row's non-zeros over the remaining lanes / (k_p / cpl) subsets,
-// folded with xor shuffles.  The shape (lanes, cpl) is chosen per k class by
-// the batch autotuner.  Same per-row arithmetic as the single-matrix CSR
-// kernels (src/compressed_sparse_rows.cpp:1114-1138 for k = 1 and the
-// row-blocked SpMM, src/compressed_sparse_rows.cpp:1699-1763, for k > 1).
+// launch can be captured in a hipGraph and replayed as is.  Inside a tile a row
+// is handled by a group of `lanes` lanes (a power of two): the k_p right-hand-side
+// columns are split over k_p / cpl lanes (cpl consecutive columns per lane, read as
+// one contiguous piece of the X row), and the row's non-zeros over the remaining
+// lanes / (k_p / cpl) subsets, folded with xor shuffles.  The shape (lanes, cpl) is
+// chosen per k class by the batch autotuner.  Same per-row arithmetic as the
+// single-matrix CSR kernels (src/compressed_sparse_rows.cpp:1114-1138 for k = 1 and
+// the row-blocked SpMM, src/compressed_sparse_rows.cpp:1699-1763, for k > 1).
 #include <algorithm>
 #include <type_traits>
 

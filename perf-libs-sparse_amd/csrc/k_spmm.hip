@@ -4,7 +4,7 @@
 // (spmm_rowwise_csr_blocked_m_kernel, src/compressed_sparse_rows.cpp:1699-1745,
 // and the C zeroing of src/matmul.cpp:596-605): beta == 0 never reads C.
 //
-// B and C are row-major (the driver lays others out again first): k_spmm_tile or
+// B and C are row-major (the entry points lay others out again first): k_spmm_tile or
 // k_spmm_lds where a block of rows shares its B rows, else k_spmm_gather.
 #include <algorithm>
 #include <type_traits>
@@ -1392,7 +1392,8 @@ void launch_bsr_mfma(const pls::DevBsr &A, int32_t k, double alpha, const void *
                      double beta, void *C, int64_t ldc, hipStream_t s) {
   constexpr int WCOLS = 4 * NB * VW * NW;  // columns of one wave
   const int32_t npass = (k + WCOLS - 1) / WCOLS;
-  constexpr int RPW = !ROWS ? 1 : sizeof(X) == 8 ? 4 / NB * bsr_rows_f64<BS, NW> : 64 / (NB * BS);  // block rows per wave
+  // block rows per wave
+  constexpr int RPW = !ROWS ? 1 : sizeof(X) == 8 ? 4 / NB * bsr_rows_f64<BS, NW> : 64 / (NB * BS);
   const int64_t units = (int64_t(A.mb) + RPW - 1) / RPW * npass, slice = int64_t(1) << 25;
   auto go = [&](auto kern) {
     for (int64_t u = 0; u < units; u += slice)
